@@ -1,0 +1,62 @@
+"""The Node128 traversal kernel where its waves share work: launches of every
+fill (one ray to more rays than lanes), so idle lanes walk subtrees of busy
+lanes' rays, against the oracle, bit for bit -- closest hit in each visiting
+order, any hit, and both with the path tracer's sided filter; and a scene of
+nearly coincident surfaces, whose near-ties a group has to walk again alone.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from vitrum_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("prim", "inst", "t", "u", "v")
+
+
+def _box():
+    return W.cornell_scene(16384)
+
+
+def _shells():
+    """Three shells of one mesh, two of them 3e-7 apart, and a second
+    instance coincident with the outer one."""
+    v, i = W.octa_sphere(8, split=True)
+    n = W._vertex_normals(v, i)
+    v3 = np.concatenate([v, v * (1 + 3e-7), v * 0.9])
+    i3 = np.concatenate([i, i + len(v), i + 2 * len(v)]).astype(np.uint32)
+    cam = W.look_at_camera(eye=(0.0, 0.3, 2.5), target=(0.0, 0.0, 0.0), up=(0, 1, 0), vfov_deg=50.0)
+    return {"primitives": [W._mesh(v3, np.concatenate([n, n, n]), i3, W.WHITE), W._mesh(v, n, i, W.RED)],
+            "camera": cam, "scene_radius": 1.0}
+
+
+@pytest.mark.parametrize("make", [_box, _shells])
+def test_every_fill_matches_oracle(engine, make):
+    sc = make()
+    engine.set_scene(sc)
+    pack = O.pack_scene([dict(p, material_id=i) for i, p in enumerate(sc["primitives"])])
+    ps = O.PackedScene(pack)
+    rays, st = W.primary_rays(sc["camera"], 256, 256, scene_radius=sc["scene_radius"])
+    rays = np.concatenate([rays, W.bounce_rays(pack, rays, O.trace_closest(ps, rays), st, sc["scene_radius"])])
+    rays = rays[np.random.default_rng(9).permutation(rays.size)]
+    seg = rays.copy()  # any-hit rays of limited length
+    seg["tmax"] = np.random.default_rng(10).uniform(0.05, 3.0, rays.size).astype(np.float32)
+    flags = O.single_sided_flags(ps, [p["material"] for p in sc["primitives"]])
+    want = {0: (O.trace_closest(ps, rays), O.trace_any(ps, seg)),
+            1: (O.trace_closest_sided(ps, flags, rays), O.trace_occluded_sided(ps, flags, seg))}
+    try:
+        # one ray; a wave less and more than full; every wave one ray; a few
+        # rays each; about a full static fill; refills from the counter
+        for n in (1, 63, 64, 65, 4095, 16411, 70001, rays.size):
+            for sided in (0, 1):
+                engine.set_hit_filter(sided)
+                for near in (0, 1, 2):
+                    engine.set_trace_tuning(8, 16, near, 12)
+                    got = engine.trace_closest(rays[:n])
+                    for k in FIELDS:
+                        assert np.array_equal(got[k].view(np.uint32), want[sided][0][k][:n].view(np.uint32)), (n, sided, near, k)
+                assert np.array_equal(engine.trace_any(seg[:n]), want[sided][1][:n]), (n, sided)
+    finally:
+        engine.set_hit_filter(0)
+        engine.set_trace_tuning(8, 16, 2, 12)

@@ -12,6 +12,9 @@
 // correctly rounded division and square root).
 //
 // Design (MI355X):
+//  * wide_kernel walks Node128 trees (four child boxes per node); scenes
+//    whose Node128 stack bound is too deep, and the work counters, take
+//    trace_kernel.
 //  * Node64 BVH2 nodes: the two child boxes sit in the parent, so a node
 //    expansion is one 64-byte load and two slab tests.  The traversal order
 //    is the reference's left-first depth-first order; a child's entry
@@ -30,7 +33,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <initializer_list>
 
 #include "traverse.h"
 #include "cwbvh.h"
@@ -85,7 +87,7 @@ __device__ __forceinline__ float edge_fn(float ax, float ay, float bx, float by)
   return ordered ? canonical : -canonical;
 }
 
-__device__ __noinline__ float ray_param(V3 o, V3 dir, V3 p) {
+__device__ __forceinline__ float ray_param_inl(V3 o, V3 dir, V3 p) {
   const V3 delta = sub(p, o);
   const float ds = max3abs(delta.x, delta.y, delta.z);
   const float rs = max3abs(dir.x, dir.y, dir.z);
@@ -97,6 +99,8 @@ __device__ __noinline__ float ray_param(V3 o, V3 dir, V3 p) {
   const float den = (d.x * d.x + d.y * d.y) + d.z * d.z;
   return (num / den) * (ds / rs);
 }
+
+__device__ __noinline__ float ray_param(V3 o, V3 dir, V3 p) { return ray_param_inl(o, dir, p); }
 
 __device__ __forceinline__ bool lex_before(V3 a, V3 b) {
   return a.x < b.x || (a.x == b.x && (a.y < b.y || (a.y == b.y && a.z < b.z)));
@@ -166,7 +170,7 @@ __device__ __forceinline__ WtRay wt_setup(V3 dir) {
 // Rare tail of an in-window hit (opticalWatertightTriangle.ts:164-220): the
 // authored-normal side test.  Returns 0 for a rejected hit, 1 for the front
 // face (side > 0), -1 for the back face.
-__device__ __noinline__ int wt_side(V3 dir, float ds, V3 a, V3 b, V3 c) {
+__device__ __forceinline__ int wt_side_inl(V3 dir, float ds, V3 a, V3 b, V3 c) {
   const V3 e1r = sub(b, a), e2r = sub(c, a);
   const float es = jmax(max3abs(e1r.x, e1r.y, e1r.z), max3abs(e2r.x, e2r.y, e2r.z));
   if (!(es > 0.0f) || !finite_(es)) return 0;
@@ -184,6 +188,8 @@ __device__ __noinline__ int wt_side(V3 dir, float ds, V3 a, V3 b, V3 c) {
   if (side == 0.0f || !finite_(side)) return 0;
   return side > 0.0f ? 1 : -1;
 }
+
+__device__ __noinline__ int wt_side(V3 dir, float ds, V3 a, V3 b, V3 c) { return wt_side_inl(dir, ds, a, b, c); }
 
 // Returns true and fills h when the triangle is hit with lo < t < hi (or
 // t <= hi when `incl_hi`), where lo = tmin (also the predicate's exclusive
@@ -329,7 +335,7 @@ __device__ __forceinline__ V3 xform_dir(float4 c0, float4 c1, float4 c2, V3 d) {
 // Node culling stays `tNear > bound` (equal distances are still visited).  The
 // counting variant always uses the reference order, so its work counts are
 // the reference's.
-template <bool ANY, bool COUNT, bool MULTI, bool W4, uint32_t BLOCK, uint32_t LDS_DEPTH>
+template <bool ANY, bool COUNT, bool MULTI, uint32_t BLOCK, uint32_t LDS_DEPTH>
 // Register budget: four waves per SIMD (128 VGPRs; with the 20-entry LDS
 // stack, 8 blocks of 128 fit a CU), which beats three waves without spills.
 __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
@@ -356,11 +362,11 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
   };
   // Scene of the current ray: the launch's scene, or (batched) the one whose
   // ray range holds the ray, looked up when the lane takes a new ray.
-  const float4* __restrict__ blas = W4 ? p.scene.blas4_nodes : p.scene.blas_nodes;
-  const float4* __restrict__ tlas = W4 ? p.scene.tlas4_nodes : p.scene.tlas_nodes;
+  const float4* __restrict__ blas = p.scene.blas_nodes;
+  const float4* __restrict__ tlas = p.scene.tlas_nodes;
   const float4* __restrict__ tris = p.scene.tris;
   const float4* __restrict__ insts = p.scene.instances;
-  uint32_t tlas_root = W4 ? p.scene.tlas4_root : p.scene.tlas_root, tlas_count = p.scene.tlas_node_count;
+  uint32_t tlas_root = p.scene.tlas_root, tlas_count = p.scene.tlas_node_count;
   const uint32_t lane = __lane_id();
   const uint64_t lane_below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const bool near = !ANY && !COUNT && p.near_first != 0u;        // inside BLASes
@@ -375,7 +381,7 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
   V3 ro{}, rd{}, rinv{};
   float tmin = 0, tmax = 0, best = 0, bu = 0, bv = 0;
   V3 bpos{};
-  uint32_t bprim = 0, binst = kMiss, bslot = 0;
+  uint32_t bprim = 0, binst = kMiss;
   bool bfront = false;  // the best hit is on the front face (world orientation)
   // near_first = 2: the lane walks in the reference's TLAS order (after a
   // near-tie), a near-tie was seen, and the magnitude of the ray origin.
@@ -427,7 +433,7 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
     inst_id = meta.y;
     level = 1;
     blas_base = sp;
-    cur = W4 ? meta.z : meta.x;
+    cur = meta.x;
     if (COUNT) ++c_inst;
   };
 
@@ -443,7 +449,6 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
         bpos = w;
         bprim = lprim;
         binst = inst_id;
-        bslot = slot;
         bu = lu;
         bv = lv;
         bfront = lfront != lmirror;
@@ -519,11 +524,11 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
               if (p.scene_offsets[mid] <= idx) lo_s = mid; else hi_s = mid;
             }
             const DeviceScene& S = p.scenes[lo_s];
-            blas = W4 ? S.blas4_nodes : S.blas_nodes;
-            tlas = W4 ? S.tlas4_nodes : S.tlas_nodes;
+            blas = S.blas_nodes;
+            tlas = S.tlas_nodes;
             tris = S.tris;
             insts = S.instances;
-            tlas_root = W4 ? S.tlas4_root : S.tlas_root;
+            tlas_root = S.tlas_root;
             tlas_count = S.tlas_node_count;
           }
           const float4 a = p.rays[2 * (size_t)idx], b = p.rays[2 * (size_t)idx + 1];
@@ -538,7 +543,6 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
           best = tmax;
           binst = kMiss;
           bprim = 0;
-          bslot = 0;
           bu = bv = 0;
           level = 0;
           sp = 0;
@@ -759,7 +763,6 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
             best = tmax;
             binst = kMiss;
             bprim = 0;
-            bslot = 0;
             bu = bv = 0.0f;
             level = 0;
             sp = 0;
@@ -778,7 +781,6 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
               best = tmax;
               binst = kMiss;
               bprim = 0;
-              bslot = 0;
               bu = bv = 0.0f;
               level = 0;
               sp = 0;
@@ -792,82 +794,7 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
         }
         if (!active || pend != kPendNone) continue;
       }
-      if (W4 && (cur & kLeafBit) == 0) {
-        // ---- interior: one Node128, four child boxes tested axis by axis ----
-        static_assert(kWideKids == 4, "the expansion below is written for 4-wide nodes");
-        const float4* nd = (level ? blas : tlas) + (size_t)kWideNodeFloat4s * cur;
-        const V3 o = level ? lo : ro;
-        const V3 inv = level ? linv : rinv;
-        const float tm = level ? ltmin : tmin;
-        const float bound = level ? lbest : world_bound();
-        float4 a = nd[0], b = nd[3];
-        float n0, n1, n2, n3, f0, f1, f2, f3;
-        {
-          const float p0 = (a.x - o.x) * inv.x, q0 = (b.x - o.x) * inv.x;
-          const float p1 = (a.y - o.x) * inv.x, q1 = (b.y - o.x) * inv.x;
-          const float p2 = (a.z - o.x) * inv.x, q2 = (b.z - o.x) * inv.x;
-          const float p3 = (a.w - o.x) * inv.x, q3 = (b.w - o.x) * inv.x;
-          n0 = fminf(p0, q0), f0 = fmaxf(p0, q0);
-          n1 = fminf(p1, q1), f1 = fmaxf(p1, q1);
-          n2 = fminf(p2, q2), f2 = fmaxf(p2, q2);
-          n3 = fminf(p3, q3), f3 = fmaxf(p3, q3);
-        }
-        a = nd[1], b = nd[4];
-        {
-          const float p0 = (a.x - o.y) * inv.y, q0 = (b.x - o.y) * inv.y;
-          const float p1 = (a.y - o.y) * inv.y, q1 = (b.y - o.y) * inv.y;
-          const float p2 = (a.z - o.y) * inv.y, q2 = (b.z - o.y) * inv.y;
-          const float p3 = (a.w - o.y) * inv.y, q3 = (b.w - o.y) * inv.y;
-          n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
-          n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
-          n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
-          n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
-        }
-        a = nd[2], b = nd[5];
-        {
-          const float p0 = (a.x - o.z) * inv.z, q0 = (b.x - o.z) * inv.z;
-          const float p1 = (a.y - o.z) * inv.z, q1 = (b.y - o.z) * inv.z;
-          const float p2 = (a.z - o.z) * inv.z, q2 = (b.z - o.z) * inv.z;
-          const float p3 = (a.w - o.z) * inv.z, q3 = (b.w - o.z) * inv.z;
-          n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
-          n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
-          n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
-          n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
-        }
-        const uint4 r = *reinterpret_cast<const uint4*>(nd + 6);
-        // The slab test of each child: !(tNear > tFar || tFar < tMin), then
-        // the bound (the pop-time cull re-checks it against the best hit).
-        const bool k0 = r.x != kEmpty && !(n0 > f0 || f0 < tm) && !(n0 > bound);
-        const bool k1 = r.y != kEmpty && !(n1 > f1 || f1 < tm) && !(n1 > bound);
-        const bool k2 = r.z != kEmpty && !(n2 > f2 || f2 < tm) && !(n2 > bound);
-        const bool k3 = r.w != kEmpty && !(n3 > f3 || f3 < tm) && !(n3 > bound);
-        if (COUNT) {
-          const uint32_t tested = (r.x != kEmpty) + (r.y != kEmpty) + (r.z != kEmpty) + (r.w != kEmpty);
-          if (level) c_blas += tested; else c_tlas += tested;
-        }
-        // Visit first: the nearest passing child (inside BLASes with
-        // near_first, lowest slot on equal distances), else the first passing
-        // slot, which is the reference's depth-first order.  The others are
-        // pushed so that they pop in slot order.
-        uint32_t first = k0 ? 0u : (k1 ? 1u : (k2 ? 2u : (k3 ? 3u : 4u)));
-        if ((level ? near : (near_tlas && !ref_order)) && first < 4u) {
-          float bt = n0;
-          bt = first == 1u ? n1 : (first == 2u ? n2 : (first == 3u ? n3 : bt));
-          if (k1 && n1 < bt) first = 1u, bt = n1;
-          if (k2 && n2 < bt) first = 2u, bt = n2;
-          if (k3 && n3 < bt) first = 3u, bt = n3;
-        }
-        bool ok = true;
-        if (k3 && first != 3u) ok = push(r.w, n3);
-        if (ok && k2 && first != 2u) ok = push(r.z, n2);
-        if (ok && k1 && first != 1u) ok = push(r.y, n1);
-        if (ok && k0 && first != 0u) ok = push(r.x, n0);
-        if (!ok) {
-          finish(false);
-          continue;
-        }
-        cur = first == 0u ? r.x : (first == 1u ? r.y : (first == 2u ? r.z : (first == 3u ? r.w : kNone)));
-      } else if (!W4 && (cur & kLeafBit) == 0) {
+      if ((cur & kLeafBit) == 0) {
         // ---- interior: one Node64 load, two child boxes ----
         const float4* nd = (level ? blas : tlas) + 4 * (size_t)cur;
         const float4 q0 = nd[0], q1 = nd[1], q2 = nd[2], q3 = nd[3];
@@ -910,6 +837,833 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Division by a shared denominator
+// ---------------------------------------------------------------------------
+
+// The correctly rounded quotient a / b from y, the refined reciprocal of b:
+// the residual-correction steps of the compiler's own expansion (two
+// remainders, each folded back with one fused multiply-add; Markstein, "IA-64
+// and Elementary Functions", 2000) without its operand scaling, which only
+// matters when a remainder or a quotient could leave the normal range.  The
+// callers check the operands with the two predicates below and divide
+// normally otherwise, so every quotient is the same bits.  Quotients that
+// share a denominator cost 6 instructions each instead of 11.
+__device__ __forceinline__ float recip_of(float b) {
+  const float y = __builtin_amdgcn_rcpf(b);
+  return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float div_by(float a, float b, float y) {
+  float q = a * y;
+  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+  return __builtin_amdgcn_div_fixupf(q, b, a);  // zeros, with their signs
+}
+__device__ __forceinline__ V3 div_by(V3 a, float b, float y) {
+  return v3(div_by(a.x, b, y), div_by(a.y, b, y), div_by(a.z, b, y));
+}
+// |x| in [2^-40, 2^40]: a denominator.
+__device__ __forceinline__ bool div_den(float x) {
+  return (f2u(x) & 0x7FFFFFFFu) - 0x2B800000u <= 0x53800000u - 0x2B800000u;
+}
+// x zero or |x| >= 2^-60, as a key: numerators are safe when the smallest of
+// their keys is at least kDivNum (zero wraps to the largest key).  With a
+// denominator below 2^40 the quotient stays above 2^-100.
+constexpr uint32_t kDivNum = (0x21800000u << 1) - 1u;
+__device__ __forceinline__ uint32_t div_key(float x) { return (f2u(x) << 1) - 1u; }
+__device__ __forceinline__ uint32_t div_key(V3 a) { return min(min(div_key(a.x), div_key(a.y)), div_key(a.z)); }
+
+// xform_point, safe_normalize and safe_inv with the shared-denominator
+// division; the general forms answer every operand outside its range.
+__device__ __forceinline__ V3 xform_point_fast(float4 c0, float4 c1, float4 c2, float4 c3, V3 p) {
+  const V3 r = v3(((c0.x * p.x + c1.x * p.y) + c2.x * p.z) + c3.x, ((c0.y * p.x + c1.y * p.y) + c2.y * p.z) + c3.y,
+                  ((c0.z * p.x + c1.z * p.y) + c2.z * p.z) + c3.z);
+  const float rw = ((c0.w * p.x + c1.w * p.y) + c2.w * p.z) + c3.w;
+  const float s = fmaxf(fmaxf(fabs_(r.x), fabs_(r.y)), fmaxf(fabs_(r.z), fabs_(rw)));
+  const float ys = recip_of(s);
+  const float qw = div_by(rw, s, ys);
+  const float sum = (r.x + r.y) + (r.z + rw);  // NaN when any of the four is
+  if (__builtin_expect(!(div_den(s) && div_den(qw) && sum == sum && min(div_key(r), div_key(rw)) >= kDivNum), 0))
+    return xform_point(c0, c1, c2, c3, p);
+  return div_by(div_by(r, s, ys), qw, recip_of(qw));
+}
+
+__device__ __forceinline__ V3 xform_dir_fast(float4 c0, float4 c1, float4 c2, V3 d) {
+  const V3 v = v3((c0.x * d.x + c1.x * d.y) + c2.x * d.z, (c0.y * d.x + c1.y * d.y) + c2.y * d.z,
+                  (c0.z * d.x + c1.z * d.y) + c2.z * d.z);
+  const float s = fmaxf(fabs_(v.x), fmaxf(fabs_(v.y), fabs_(v.z)));
+  if (__builtin_expect(!(div_den(s) && div_key(v) >= kDivNum), 0)) return safe_normalize(v);
+  const V3 q = div_by(v, s, recip_of(s));
+  const float len = __builtin_sqrtf((q.x * q.x + q.y * q.y) + q.z * q.z);  // in [1, sqrt 3]
+  return div_by(q, len, recip_of(len));
+}
+
+__device__ __forceinline__ V3 safe_inv3(V3 v) {
+  if (__builtin_expect(!(div_den(v.x) && div_den(v.y) && div_den(v.z)), 0))
+    return v3(safe_inv(v.x), safe_inv(v.y), safe_inv(v.z));
+  return v3(div_by(1.0f, v.x, recip_of(v.x)), div_by(1.0f, v.y, recip_of(v.y)), div_by(1.0f, v.z, recip_of(v.z)));
+}
+
+// The watertight test of one (ray, triangle) pair, as tri_test: the same
+// operations in the same order, with the divisions by the determinant and
+// by the edge and normal scales shared, and the rare zero-edge cases inline.
+__device__ __forceinline__ bool pair_test(V3 o, V3 dir, const WtRay& w, V3 a, V3 b, V3 c, float tmin, float hi,
+                                          bool incl_hi, TriHit& h) {
+  const int kx = w.perm & 3, ky = (w.perm >> 2) & 3, kz = (w.perm >> 4) & 3;
+  const V3 pa = sub(a, o), pb = sub(b, o), pc = sub(c, o);
+  const float paz = sel3(kz, pa.x, pa.y, pa.z), pbz = sel3(kz, pb.x, pb.y, pb.z), pcz = sel3(kz, pc.x, pc.y, pc.z);
+  const float apx = sel3(kx, pa.x, pa.y, pa.z) - w.sx * paz, apy = sel3(ky, pa.x, pa.y, pa.z) - w.sy * paz;
+  const float bpx = sel3(kx, pb.x, pb.y, pb.z) - w.sx * pbz, bpy = sel3(ky, pb.x, pb.y, pb.z) - w.sy * pbz;
+  const float cpx = sel3(kx, pc.x, pc.y, pc.z) - w.sx * pcz, cpy = sel3(ky, pc.x, pc.y, pc.z) - w.sy * pcz;
+  const float e0 = edge_fn(bpx, bpy, cpx, cpy);
+  const float e1 = edge_fn(cpx, cpy, apx, apy);
+  const float e2 = edge_fn(apx, apy, bpx, bpy);
+  const float det = (e0 + e1) + e2;
+  if (w.perm == 0xFFFFFFFFu || nan_(tmin) || det == 0.0f || !finite_(det)) return false;
+  const bool positive = det > 0.0f;
+  const float n0 = positive ? e0 : -e0, n1 = positive ? e1 : -e1, n2 = positive ? e2 : -e2;
+  if (n0 < 0.0f || n1 < 0.0f || n2 < 0.0f) return false;
+  const float scaled_t = (e0 * (paz * w.sz) + e1 * (pbz * w.sz)) + e2 * (pcz * w.sz);
+  const int zc = (n0 == 0.0f) + (n1 == 0.0f) + (n2 == 0.0f);
+  float t;
+  V3 point = v3(0, 0, 0);
+  if (__builtin_expect(zc != 0, 0)) {
+    // On an edge or a vertex (opticalWatertightTriangle.ts:120-160): the
+    // canonical point of the shared edge, or the vertex itself.
+    bool ok = true;
+    if (zc >= 2) {
+      if (n0 != 0.0f) point = a;
+      if (n1 != 0.0f) point = b;
+      if (n2 != 0.0f) point = c;
+    } else {
+      const bool on0 = n0 == 0.0f, on1 = n1 == 0.0f;
+      const V3 fi = on0 ? b : (on1 ? c : a), si = on0 ? c : (on1 ? a : b);
+      const float fx = on0 ? bpx : (on1 ? cpx : apx), fy = on0 ? bpy : (on1 ? cpy : apy);
+      const float gx = on0 ? cpx : (on1 ? apx : bpx), gy = on0 ? cpy : (on1 ? apy : bpy);
+      const bool ordered = lex_before(fi, si);
+      const V3 f = ordered ? fi : si, s = ordered ? si : fi;
+      const float ax = ordered ? fx : gx, ay = ordered ? fy : gy;
+      const float ddx = (ordered ? gx : fx) - ax, ddy = (ordered ? gy : fy) - ay;
+      const bool use_x = fabs_(ddx) >= fabs_(ddy);
+      const float num = use_x ? -ax : -ay, den = use_x ? ddx : ddy;
+      ok = den != 0.0f;
+      const float q = num / (ok ? den : 1.0f);
+      point = ok ? v3(f.x + q * (s.x - f.x), f.y + q * (s.y - f.y), f.z + q * (s.z - f.z)) : point;
+    }
+    t = ok ? ray_param_inl(o, dir, point) : -1.0f;
+  }
+  const float yd = recip_of(det);
+  const bool fast = div_den(det * 0x1p20f) && div_den(w.ds) && fabs_(scaled_t) < 0x1p40f &&
+                    min(min(div_key(scaled_t), div_key(e1)), div_key(e2)) >= kDivNum;
+  if (zc == 0) {
+    if (__builtin_expect(fast, 1)) {
+      const float t1 = div_by(scaled_t, det, yd);
+      t = div_key(t1) >= kDivNum ? div_by(t1, w.ds, recip_of(w.ds)) : t1 / w.ds;
+    } else {
+      t = (scaled_t / det) / w.ds;
+    }
+  }
+  const float lo = tmin > 0.0f ? tmin : 0.0f;
+  if (!(t > lo) || !finite_(t)) return false;
+  if (!(t > tmin && (t < hi || (incl_hi && t == hi)))) return false;
+  // The authored-normal side test (opticalWatertightTriangle.ts:164-219).
+  const V3 e1r = sub(b, a), e2r = sub(c, a);
+  const float es = fmaxf(fmaxf(fmaxf(fabs_(e1r.x), fabs_(e1r.y)), fmaxf(fabs_(e1r.z), fabs_(e2r.x))),
+                         fmaxf(fabs_(e2r.y), fabs_(e2r.z)));
+  int side;
+  const float ye = recip_of(es);
+  const V3 s1 = div_by(e1r, es, ye), s2 = div_by(e2r, es, ye);
+  const V3 nr = v3(s1.y * s2.z - s1.z * s2.y, s1.z * s2.x - s1.x * s2.z, s1.x * s2.y - s1.y * s2.x);
+  const float ns = fmaxf(fabs_(nr.x), fmaxf(fabs_(nr.y), fabs_(nr.z)));
+  const bool side_fast = div_den(es) && div_den(ns) && div_den(w.ds) &&
+                         min(min(div_key(e1r), div_key(e2r)), min(div_key(nr), div_key(dir))) >= kDivNum;
+  if (__builtin_expect(side_fast, 1)) {
+    const V3 nd = div_by(nr, ns, recip_of(ns));
+    const float nl = __builtin_sqrtf((nd.x * nd.x + nd.y * nd.y) + nd.z * nd.z);  // in [1, sqrt 3]
+    const V3 n = div_by(nd, nl, recip_of(nl));
+    const V3 d = div_by(dir, w.ds, recip_of(w.ds));
+    const float sd = -((d.x * n.x + d.y * n.y) + d.z * n.z);
+    side = sd == 0.0f ? 0 : (sd > 0.0f ? 1 : -1);
+  } else {
+    side = wt_side_inl(dir, w.ds, a, b, c);
+  }
+  if (side == 0) return false;
+  h.front = side > 0;
+  h.t = t;
+  h.u = fast ? div_by(e1, det, yd) : e1 / det;
+  h.v = fast ? div_by(e2, det, yd) : e2 / det;
+  h.point = zc == 0 ? v3(a.x + (h.u * (b.x - a.x) + h.v * (c.x - a.x)), a.y + (h.u * (b.y - a.y) + h.v * (c.y - a.y)),
+                         a.z + (h.u * (b.z - a.z) + h.v * (c.z - a.z)))
+                    : point;
+  return true;
+}
+
+// ---------------------------------------------------------------------------
+// Persistent traversal of the Node128 trees
+// ---------------------------------------------------------------------------
+
+// The walk of trace_kernel over the 4-wide trees: the same boxes, triangles,
+// tests and acceptance rules, so the same hit records.
+//
+// What bounds it is VALU issue (a wave's lanes diverge) and, at the end of a
+// launch, the serial chain of its longest rays.  Three things follow.
+//
+// One current ray.  Origin, reciprocal direction, lower bound, cull bound and
+// node array are those of the level a lane walks; an instance exit reloads
+// the world ray from memory instead of keeping both in registers (and nothing
+// selects between them in each step).  A ray's record is written when an
+// instance improves it, so its prim, u, v and position take no registers.
+//
+// Divisions share their denominators (div_by).
+//
+// Lanes without a ray help.  Once a wave has no rays left to fetch, an idle
+// lane takes the bottom entry of a busy lane's BLAS stack -- the largest
+// subtree it has not begun -- with a copy of its local ray, and walks it as
+// if it were its own.  The lane that entered the instance (the owner) waits
+// at the instance's exit until all its helpers are done and takes the
+// smallest (t, triangle) over them.  The group shares its best distance
+// through LDS.  A helped closest-hit walk visits boxes in another order, and
+// the order matters where two triangles are hit within the rounding of the
+// box tests: so a group culls against its best distance plus a margin
+// (2^-13 of the distance and the origin's magnitude, as for instances), and
+// when two hits come within that margin the owner walks the instance again
+// alone, in the usual order.  Without such a near-tie the nearest triangle is
+// never culled in any order, and it is the one that any order keeps.  Any-hit
+// answers do not depend on the order at all.
+//
+// Measured against the same walk without these three (trace_kernel over
+// Node128): 1,677,721 rays of the 1M-triangle scene 1.294 -> 0.944 ms;
+// 419,430 rays of the 32,768-triangle box, one launch after another on three
+// streams, 0.356 -> 0.157 ms and alone 0.99 -> 0.43 ms (its longest ray takes
+// 322 steps, most rays under 60); a 256 x 256 path-traced frame of that box
+// (17 launches of at most 65,536 rays) 7.6 -> 3.1 ms.
+constexpr uint32_t kIdle = 0, kNode = 1, kLeaf = 2, kEnter = 3, kExit = 4, kDone = 5;  // what a lane does next
+constexpr uint32_t kfHit = 1u;         // the record holds a hit
+constexpr uint32_t kfReject = 2u;      // ... on the back face of a single-sided material
+constexpr uint32_t kfRefOrder = 4u;    // walking the TLAS in the reference's order
+constexpr uint32_t kfRecheck = 8u;     // two instances' hits came within the margin
+constexpr uint32_t kfLevel = 16u;      // inside an instance
+constexpr uint32_t kfMirror = 32u;     // ... whose local-to-world map reverses orientation
+constexpr uint32_t kfWt = 64u;         // the watertight set-up of the local ray is done
+constexpr uint32_t kfLHit = 128u;      // local hit, and its two bits
+constexpr uint32_t kfLFront = 256u;
+constexpr uint32_t kfLSingle = 512u;
+constexpr uint32_t kfSplit = 1024u;    // in a group: an owner with helpers, or a helper
+constexpr uint32_t kfHelper = 2048u;
+constexpr uint32_t kfTie = 4096u;      // two hits of the group came within the margin
+constexpr uint32_t kfAlone = 8192u;    // no helpers in this instance (walked again after a near-tie)
+constexpr uint32_t kfLocal = kfLevel | kfMirror | kfWt | kfLHit | kfLFront | kfLSingle | kfSplit | kfTie;
+constexpr uint32_t kHelpSteps = 4;     // steps between two rounds of taking work
+
+// Orders a wave's LDS accesses of different lanes (they execute in program
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <bool ANY, bool MULTI>
+// Four waves per SIMD: 128 VGPRs, and 8 blocks of 128 fit a CU's LDS.
+__global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
+  constexpr uint32_t B = kTraceBlock, D = kWideLdsDepth;
+  // Stack entries (child ref, entry distance), entry-major, deeper ones in a
+  // per-thread global area; per wave: the pair table of a leaf operation
+  // (also the donors' lanes), the groups' best distances and helper counts.
+  __shared__ uint32_t st_ref[D * B];
+  __shared__ float st_tn[D * B];
+  __shared__ uint32_t table[B], group_best[B], helpers[B];
+  const uint32_t tid = threadIdx.x, lane = __lane_id(), wbase = tid & ~63u;
+  const size_t spill_stride = (size_t)gridDim.x * B, gtid = (size_t)blockIdx.x * B + tid;
+  unsigned long long* __restrict__ spill = reinterpret_cast<unsigned long long*>(p.spill);
+  const uint64_t lane_below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const bool near = !ANY && p.near_first != 0u;
+  const bool near_tlas = !ANY && p.near_first == 2u;
+  helpers[tid] = 0u;
+
+  const uint32_t n_rays = p.n_ptr ? *p.n_ptr : p.n;
+  const uint32_t n_waves = gridDim.x * (B / 64u);
+  const uint32_t take_cap = max(1u, min(64u, n_rays / n_waves + (n_rays % n_waves != 0u)));
+  const uint32_t wave_id = blockIdx.x * (B / 64u) + tid / 64u;
+  const uint32_t static_end = n_waves * take_cap;
+
+  uint32_t mode = kIdle, fl = 0, ray_idx = 0, sid = 0;
+  // The current level's ray: origin, reciprocal direction, lower bound, cull
+  // bound and nodes.  World: `best` (any hit: tMax) and the lower bound.
+  V3 o{}, inv{};
+  float tlow = 0, cullb = 0, best = 0, wlow = 0;
+  const float4* nodes = nullptr;
+  // Local: direction, watertight set-up, best hit, the bound it entered with.
+  V3 ld{}, lpos{};
+  WtRay lw{};
+  float lbest = 0, lcap = 0, lu = 0, lv = 0;
+  uint32_t lprim = 0, slot = 0, slot_end = 0, own = lane;
+  uint32_t cur = kNone, sp = 0, base = 0, tsp = 0;  // stack: next entry, the level's first, the TLAS part's end
+
+  auto scene_of = [&]() -> const DeviceScene& { return MULTI ? p.scenes[sid] : p.scene; };
+  auto margin = [&](float t) { return (t + max(fabs_(o.x), max(fabs_(o.y), fabs_(o.z)))) * 0x1p-13f; };
+  // The TLAS walk's bound (o is the world origin), widened by the near-tie
+  // margin while the lane orders the TLAS by distance.
+  auto world_bound = [&]() -> float {
+    if (!ANY && near_tlas && (fl & (kfHit | kfRefOrder)) == kfHit) return best + margin(best);
+    return best;
+  };
+  auto stk_load = [&](uint32_t i) -> uint2 {
+    if (i < D) return make_uint2(st_ref[i * B + tid], f2u(st_tn[i * B + tid]));
+    const unsigned long long w = spill[(i - D) * spill_stride + gtid];
+    return make_uint2((uint32_t)w, (uint32_t)(w >> 32));
+  };
+  auto finish = [&](bool occluded) {
+    if (ANY) {
+      p.occluded[ray_idx] = occluded ? 1u : 0u;
+    } else if (!(fl & kfHit)) {
+      uint32_t* h = p.hits + 5 * (size_t)ray_idx;
+      h[0] = h[1] = kMiss;
+      h[2] = 0x7F800000u;
+      h[3] = h[4] = 0u;
+      if (p.hit_pos) {
+        float* hp = p.hit_pos + 3 * (size_t)ray_idx;
+        hp[0] = hp[1] = hp[2] = 0.0f;
+      }
+    }
+    mode = kIdle;
+  };
+  // From the TLAS root with the interval (wlow, best); o and inv are the world ray's.
+  auto restart = [&]() {
+    fl &= ~(kfHit | kfReject);
+    tlow = wlow;
+    cullb = best;
+    sp = base = 0;
+    cur = MULTI ? p.scenes[sid].tlas4_root : p.scene.tlas4_root;
+    mode = kNode;
+  };
+  // A lane's subtree or interval is done: the next entry that its bound keeps.
+  auto pop = [&]() {
+    for (;;) {
+      if (sp > base) {
+        const uint2 e = stk_load(--sp);
+        if (u2f(e.y) > cullb) continue;
+        cur = e.x;
+        return;
+      }
+      if (fl & kfLevel) {
+        mode = (fl & kfHelper) ? kDone : kExit;
+        return;
+      }
+      if (!ANY && (fl & kfRecheck)) {
+        // A near-tie between instances: walk the ray again, from its
+        // original interval, in the reference's TLAS order.
+        wlow = p.rays[2 * (size_t)ray_idx].w;
+        best = p.rays[2 * (size_t)ray_idx + 1].w;
+        fl = (fl & ~kfRecheck) | kfRefOrder;
+        restart();
+        return;
+      }
+      // traceClosest (intersection.wgsl.ts:462-490): a back-face hit on a
+      // single-sided material is not a surface; the trace starts again
+      // with its distance as the exclusive lower bound, and ends as a
+      // miss once that bound stops advancing or reaches tMax.
+      if (!ANY && (fl & kfReject)) {
+        const float tmax = p.rays[2 * (size_t)ray_idx + 1].w;
+        if (best > wlow && best < tmax) {
+          wlow = best;
+          best = tmax;
+          restart();
+          return;
+        }
+        fl &= ~kfHit;
+      }
+      finish(false);
+      return;
+    }
+  };
+
+  // The first fill is static, later ones go through the shared counter (see
+  // trace_kernel); `exhausted`: no more rays for this wave.
+  bool exhausted = false, first_fill = true;
+  for (;;) {
+    const uint64_t idle = __ballot(mode == kIdle);
+    const uint32_t n_idle = (uint32_t)__popcll(idle);
+    if (!exhausted) {
+      if (n_idle >= p.refill_min || n_idle == 64u) {
+        const uint32_t take = min(n_idle, take_cap);
+        uint32_t first = wave_id * take_cap;
+        if (!first_fill) {
+          if (lane == 0) first = static_end + atomicAdd(p.counter, take);
+          first = (uint32_t)__shfl((int)first, 0);
+        }
+        first_fill = false;
+        exhausted = first + take >= n_rays;
+        const uint32_t rank = (uint32_t)__popcll(idle & lane_below), idx = first + rank;
+        if (mode == kIdle && rank < take && idx < n_rays) {
+          ray_idx = idx;
+          if (MULTI) {
+            uint32_t lo_s = 0, hi_s = p.scene_count;
+            while (lo_s + 1u < hi_s) {
+              const uint32_t mid = (lo_s + hi_s) >> 1;
+              if (p.scene_offsets[mid] <= idx) lo_s = mid; else hi_s = mid;
+            }
+            sid = lo_s;
+          }
+          const float4 a = p.rays[2 * (size_t)idx], b = p.rays[2 * (size_t)idx + 1];
+          const DeviceScene& S = scene_of();
+          nodes = S.tlas4_nodes;
+          o = v3(a.x, a.y, a.z);
+          inv = safe_inv3(v3(b.x, b.y, b.z));
+          wlow = a.w;
+          best = b.w;
+          fl = 0;
+          own = lane;
+          restart();
+          if (S.tlas_node_count == 0u) finish(false);  // no TLAS: fail closed
+        }
+      }
+    } else if (idle != 0ull && n_idle != 64u) {
+      // ---- share the groups' bounds, then hand out work ----
+      if (mode == kIdle) fl = 0;
+      if (!ANY && (fl & kfSplit)) {
+        if (fl & kfLHit) atomicMin(&group_best[wbase + own], f2u(lbest));  // t > 0: ordered as integers
+      }
+      wave_sync();
+      if (!ANY && (fl & kfSplit)) {
+        const float g = u2f(group_best[wbase + own]);
+        cullb = fminf(cullb, g + margin(g));
+      }
+      const bool donor = (fl & (kfLevel | kfAlone)) == kfLevel && (mode == kNode || mode == kLeaf) && sp > base && base < D;
+      const uint64_t donors = __ballot(donor);
+      if (donors != 0ull) {
+        // The r-th idle lane takes entry r / n_donors of donor r % n_donors.
+        const uint32_t n_don = (uint32_t)__popcll(donors), rank_d = (uint32_t)__popcll(donors & lane_below);
+        const uint32_t avail = donor ? min(sp, D) - base : 0u;
+        if (donor) table[wbase + rank_d] = lane;
+        wave_sync();
+        const uint32_t r = (uint32_t)__popcll(idle & lane_below), k = r / n_don;
+        const int d = mode == kIdle ? (int)table[wbase + (r - k * n_don)] : (int)lane;
+        wave_sync();
+        const uint32_t d_avail = (uint32_t)__shfl((int)avail, d);
+        const bool got = mode == kIdle && k < d_avail;
+        const uint32_t at = (uint32_t)__shfl((int)base, d) + k;
+        const uint32_t d_own = (uint32_t)__shfl((int)own, d), d_fl = (uint32_t)__shfl((int)fl, d);
+        const V3 d_o = v3(__shfl(o.x, d), __shfl(o.y, d), __shfl(o.z, d));
+        const V3 d_inv = v3(__shfl(inv.x, d), __shfl(inv.y, d), __shfl(inv.z, d));
+        const V3 d_ld = v3(__shfl(ld.x, d), __shfl(ld.y, d), __shfl(ld.z, d));
+        const float d_low = __shfl(tlow, d), d_cull = __shfl(cullb, d), d_cap = __shfl(lcap, d);
+        const uint64_t d_nodes = (uint64_t)(uintptr_t)nodes;
+        const uint32_t d_nlo = (uint32_t)__shfl((int)(uint32_t)d_nodes, d);
+        const uint32_t d_nhi = (uint32_t)__shfl((int)(uint32_t)(d_nodes >> 32), d);
+        const uint32_t d_sid = MULTI ? (uint32_t)__shfl((int)sid, d) : 0u;
+        if (donor) {
+          const uint32_t share = n_idle > rank_d ? (n_idle - rank_d - 1u) / n_don + 1u : 0u;
+          base += min(avail, share);
+          if (share != 0u && !(fl & kfSplit)) {
+            fl |= kfSplit;
+            if (!ANY) group_best[tid] = (fl & kfLHit) ? f2u(lbest) : 0x7F7FFFFFu;
+          }
+        }
+        wave_sync();
+        if (got) {
+          const uint32_t ref = st_ref[at * B + wbase + (uint32_t)d];
+          const float tn = st_tn[at * B + wbase + (uint32_t)d];
+          own = d_own;
+          o = d_o;
+          inv = d_inv;
+          ld = d_ld;
+          tlow = d_low;
+          cullb = d_cull;
+          lcap = d_cap;
+          nodes = reinterpret_cast<const float4*>((uintptr_t)(((uint64_t)d_nhi << 32) | d_nlo));
+          sid = d_sid;
+          fl = kfHelper | kfSplit | kfLevel | (d_fl & kfMirror);
+          lbest = d_cap;
+          sp = base = tsp = 0;
+          cur = tn > cullb ? kNone : ref;
+          mode = (cur != kNone && (cur & kLeafBit)) ? kLeaf : kNode;
+          atomicAdd(&helpers[wbase + own], 1u);
+        }
+      }
+    }
+    if (!__any(mode != kIdle)) break;
+
+    const uint32_t n_steps = exhausted ? kHelpSteps : p.steps;
+    for (uint32_t step = 0; step < n_steps; ++step) {
+      if (exhausted) {
+        // ---- helpers that are done ----
+        uint64_t done = __ballot(mode == kDone);
+        if (done) {
+          uint64_t found = __ballot(mode == kDone && (fl & (kfLHit | kfTie)));
+          if (mode == kDone) {
+            atomicSub(&helpers[wbase + own], 1u);
+            mode = kIdle;
+          }
+          while (found) {
+            const int h = __ffsll((unsigned long long)found) - 1;
+            found &= found - 1ull;
+            const uint32_t ho = (uint32_t)__builtin_amdgcn_readlane((int)own, h);
+            if (ANY) {
+              // occluded: the owner is done, and so is every lane of its group
+              const bool mine = lane == ho && mode != kIdle && own == lane;
+              if (mine) finish(true);
+              if ((fl & kfHelper) && own == ho) mode = kIdle;
+              found &= __ballot(!((fl & kfHelper) && own == ho));
+              if (lane == ho) helpers[tid] = 0u;
+            } else {
+              const uint32_t hf = (uint32_t)__builtin_amdgcn_readlane((int)fl, h);
+              const float ht = u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(lbest), h));
+              const uint32_t hprim = (uint32_t)__builtin_amdgcn_readlane((int)lprim, h);
+              const float hu = u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(lu), h));
+              const float hv = u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(lv), h));
+              const V3 hp = v3(u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(lpos.x), h)),
+                               u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(lpos.y), h)),
+                               u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(lpos.z), h)));
+              if (lane == ho) {
+                fl |= hf & kfTie;
+                if (hf & kfLHit) {
+                  if ((fl & kfLHit) && fabs_(ht - lbest) <= margin(fminf(ht, lbest))) fl |= kfTie;
+                  if (!(fl & kfLHit) || ht < lbest) {
+                    fl = (fl & ~(kfLFront | kfLSingle)) | kfLHit | (hf & (kfLFront | kfLSingle));
+                    lbest = ht;
+                    lprim = hprim;
+                    lu = hu;
+                    lv = hv;
+                    lpos = hp;
+                    cullb = fminf(lcap, ht + margin(ht));
+                  }
+                }
+              }
+            }
+          }
+        }
+      }
+      // ---- deferred work, shared by the lanes that need it (see trace_kernel) ----
+      const uint64_t m_pend = __ballot(mode >= kLeaf && mode <= kExit);
+      const uint64_t m_cheap = __ballot(mode == kNode);
+      if ((m_pend | m_cheap) == 0ull) break;
+      const uint32_t dm = min(p.defer_min, ((uint32_t)__popcll(m_pend | m_cheap) + 1u) >> 1);
+      if (m_cheap == 0ull || (uint32_t)__popcll(m_pend) >= dm) {
+        const bool all = m_cheap == 0ull;
+        const bool at_exit = mode == kExit && !((fl & kfSplit) && helpers[tid] != 0u);
+        const uint64_t m_exit = __ballot(at_exit);
+        const uint64_t m_enter = __ballot(mode == kEnter);
+        const uint64_t m_leaf = __ballot(mode == kLeaf);
+        if (all && (m_exit | m_enter | m_leaf) == 0ull) {
+          // Only owners that wait, and no helper to wait for: cannot happen.
+          // Report it and end the wave rather than wait for ever.
+          if (lane == 0) atomicOr(p.error, 2u);
+          mode = kIdle;
+          break;
+        }
+        if (m_exit && (all || (uint32_t)__popcll(m_exit) >= dm) && at_exit) {
+          mode = kNode;
+          cur = kNone;
+          sp = tsp;
+          base = 0;
+          if (!ANY && (fl & kfTie)) {
+            // a near-tie inside the group: this instance again, alone
+            fl = (fl & ~kfLocal) | kfAlone;
+            mode = kEnter;
+          } else {
+            const DeviceScene& S = scene_of();
+            const float4 a = p.rays[2 * (size_t)ray_idx], b = p.rays[2 * (size_t)ray_idx + 1];
+            const V3 rd = v3(b.x, b.y, b.z);
+            const bool hit = !ANY && (fl & kfLHit) && lbest > tlow;
+            o = v3(a.x, a.y, a.z);
+            inv = safe_inv3(rd);
+            nodes = S.tlas4_nodes;
+            if (hit) {
+              const float4* ir = S.instances + 9 * (size_t)slot + 4;
+              const float4 c0 = ir[0], c1 = ir[1], c2 = ir[2], c3 = ir[3];
+              const uint32_t inst = reinterpret_cast<const uint4*>(ir + 4)->y;
+              const V3 w = xform_point_fast(c0, c1, c2, c3, lpos);
+              const float wd = dot3(sub(w, o), rd);
+              if (near_tlas && (fl & (kfHit | kfRefOrder)) == kfHit && fabsf(wd - best) <= margin(best)) fl |= kfRecheck;
+              if (wd > wlow && wd < best) {
+                const bool front = ((fl & kfLFront) != 0u) != ((fl & kfMirror) != 0u);
+                best = wd;
+                fl = (fl & ~kfReject) | kfHit | (p.sided && !front && (fl & kfLSingle) ? kfReject : 0u);
+                uint32_t* h = p.hits + 5 * (size_t)ray_idx;
+                h[0] = lprim;
+                h[1] = inst;
+                h[2] = f2u(wd);
+                h[3] = f2u(lu);
+                h[4] = f2u(lv);
+                if (p.hit_pos) {
+                  float* hp = p.hit_pos + 3 * (size_t)ray_idx;
+                  hp[0] = w.x;
+                  hp[1] = w.y;
+                  hp[2] = w.z;
+                }
+              }
+            }
+            fl &= ~(kfLocal | kfAlone);
+            tlow = wlow;
+            cullb = world_bound();
+            if (++slot < slot_end) mode = kEnter;
+          }
+        }
+        if (m_enter && (all || (uint32_t)__popcll(m_enter) >= dm) && mode == kEnter) {
+          const DeviceScene& S = scene_of();
+          const float4* ir = S.instances + 9 * (size_t)slot;
+          const float4 a = p.rays[2 * (size_t)ray_idx], b = p.rays[2 * (size_t)ray_idx + 1];
+          const float4 c0 = ir[0], c1 = ir[1], c2 = ir[2], c3 = ir[3];
+          const uint4 meta = *reinterpret_cast<const uint4*>(ir + 8);
+          const V3 ro = v3(a.x, a.y, a.z), rd = v3(b.x, b.y, b.z);
+          o = ro;
+          const float bound = ANY ? best : world_bound();
+          const V3 lo = xform_point_fast(c0, c1, c2, c3, ro);
+          ld = xform_dir_fast(c0, c1, c2, rd);
+          const V3 start = v3(ro.x + rd.x * wlow, ro.y + rd.y * wlow, ro.z + rd.z * wlow);
+          tlow = fmaxf(dot3(sub(xform_point_fast(c0, c1, c2, c3, start), lo), ld), 0.0f);
+          // Closest: localTMax starts at INFINITY; any-hit: at the ray's tMax
+          // (tlasSceneHitTraversal.wgsl.ts:103-108 and :168-173).
+          lcap = ANY ? best : inf_const();
+          if (bound < inf_const() * 0.5f) {
+            const V3 end = v3(ro.x + rd.x * bound, ro.y + rd.y * bound, ro.z + rd.z * bound);
+            lcap = fmaxf(dot3(sub(xform_point_fast(c0, c1, c2, c3, end), lo), ld), tlow);
+          }
+          o = lo;
+          inv = safe_inv3(ld);
+          lbest = cullb = lcap;
+          fl = (fl & ~kfLocal) | kfLevel | (meta.w != 0u ? kfMirror : 0u);
+          nodes = S.blas4_nodes;
+          tsp = base = sp;
+          cur = meta.z;
+          mode = kNode;
+        }
+        if (m_leaf && (all || (uint32_t)__popcll(m_leaf) >= dm)) {
+          // The leaves' (ray, triangle) pairs are spread over all 64 lanes,
+          // 64 pairs a round; every pair is tested against its ray's state at
+          // the start of the round, then each ray keeps the smallest
+          // (t, triangle index) of its pairs -- what testing them one after
+          // another gives.
+          const bool mine = mode == kLeaf;
+          uint32_t cnt = 0;
+          const uint32_t tfirst = cur & 0x07FFFFFFu;
+          if (mine) {
+            cnt = (cur >> 27) & 15u;
+            cur = kNone;
+            mode = kNode;
+            if (!(fl & kfWt)) {
+              lw = wt_setup(ld);
+              fl |= kfWt;
+            }
+          }
+          uint32_t excl = 0, total = 0;
+#pragma unroll
+          for (uint32_t b = 0; b < 4; ++b) {  // counts are below 16: one ballot per bit
+            const uint64_t m = __ballot((cnt >> b) & 1u);
+            excl += (uint32_t)__popcll(m & lane_below) << b;
+            total += (uint32_t)__popcll(m) << b;
+          }
+          bool occl = false;
+          for (uint32_t first = 0; first < total; first += 64u) {
+            uint32_t most = 0;  // the largest count
+            for (; __ballot(most < cnt) != 0ull; ++most) {
+              const uint32_t q = excl + most - first;
+              if (most < cnt && q < 64u) table[wbase + q] = lane | (most << 8);
+            }
+            wave_sync();
+            const bool work = first + lane < total;
+            const uint32_t entry = work ? table[wbase + lane] : lane;
+            wave_sync();
+            const int ol = (int)(entry & 63u);
+            const uint32_t tri = (uint32_t)__shfl((int)tfirst, ol) + (entry >> 8);
+            const V3 wo = v3(__shfl(o.x, ol), __shfl(o.y, ol), __shfl(o.z, ol));
+            const V3 wd = v3(__shfl(ld.x, ol), __shfl(ld.y, ol), __shfl(ld.z, ol));
+            WtRay ww;
+            ww.ds = __shfl(lw.ds, ol);
+            ww.sx = __shfl(lw.sx, ol);
+            ww.sy = __shfl(lw.sy, ol);
+            ww.sz = __shfl(lw.sz, ol);
+            ww.perm = (uint32_t)__shfl((int)lw.perm, ol);
+            const float w_low = __shfl(tlow, ol);
+            // An owner or helper accepts up to its cull bound (its best plus
+            // the margin); otherwise hits below the best, or at it.
+            const float w_hi = __shfl((fl & kfSplit) ? cullb : lbest, ol);
+            const uint32_t w_fl = (uint32_t)__shfl((int)fl, ol);
+            const float4* otris = p.scene.tris;
+            if (MULTI) otris = p.scenes[(uint32_t)__shfl((int)sid, ol)].tris;
+            TriHit h;
+            h.t = h.u = h.v = 0.0f;
+            h.point = v3(0, 0, 0);
+            h.front = false;
+            bool hit = false;
+            float single = 0.0f;
+            if (work) {
+              const float4* tr = otris + 3 * (size_t)tri;
+              const float4 w0 = tr[0], w1 = tr[1], w2 = tr[2];
+              single = w2.y;
+              hit = pair_test(wo, wd, ww, v3(w0.x, w0.y, w0.z), v3(w0.w, w1.x, w1.y), v3(w1.z, w1.w, w2.x), w_low, w_hi,
+                              near && (w_fl & (kfLHit | kfSplit)) == kfLHit, h);
+              // Any hit through the path tracer's wrappers: a back face of a
+              // single-sided material does not block.
+              if (ANY && hit && p.sided && h.front == ((w_fl & kfMirror) != 0u) && single > 0.5f) hit = false;
+            }
+            const uint64_t hits = __ballot(hit);
+            if (hits == 0ull) continue;
+            // Each ray's run of lanes in this round: [lo, hi).
+            const uint32_t lo = min(max(excl, first) - first, 64u), hi = min(max(excl + cnt, first) - first, 64u);
+            const uint64_t run = (hi > lo) ? ((~0ull >> (64u - (hi - lo))) << lo) & hits : 0ull;
+            if (ANY) {
+              occl = occl || run != 0ull;
+              continue;
+            }
+            float rt = __builtin_inff();
+            uint32_t rl = lane, ri = 0;
+            for (uint32_t i = 0; i < most; ++i) {
+              const uint32_t q = excl + i - first;
+              const float t = __shfl(h.t, (int)(q & 63u));
+              if (i < cnt && q < 64u && ((hits >> (q & 63u)) & 1ull) && t < rt) {
+                rt = t;
+                rl = q;
+                ri = tfirst + i;
+              }
+            }
+            const uint32_t bits = (h.front ? kfLFront : 0u) | (single > 0.5f ? kfLSingle : 0u);
+            const float ru = __shfl(h.u, (int)rl), rv = __shfl(h.v, (int)rl);
+            const V3 rp = v3(__shfl(h.point.x, (int)rl), __shfl(h.point.y, (int)rl), __shfl(h.point.z, (int)rl));
+            const uint32_t rb = (uint32_t)__shfl((int)bits, (int)rl);
+            if (run != 0ull) {
+              if (fl & kfSplit) {
+                // two hits in one leaf, or one within the margin of the best
+                if ((run & (run - 1ull)) != 0ull) fl |= kfTie;
+                if ((fl & kfLHit) && fabs_(rt - lbest) <= margin(fminf(rt, lbest))) fl |= kfTie;
+              }
+              if (!(fl & kfLHit) || rt < lbest || (rt == lbest && ri < lprim)) {
+                fl = (fl & ~(kfLFront | kfLSingle)) | kfLHit | rb;
+                lbest = rt;
+                lprim = ri;
+                lu = ru;
+                lv = rv;
+                lpos = rp;
+                cullb = (fl & kfSplit) ? fminf(cullb, fminf(lcap, rt + margin(rt))) : rt;
+              }
+            }
+          }
+          if (ANY && occl) {
+            // A group's lanes end together, at the owner.
+            if (!(fl & kfSplit)) {
+              finish(true);
+            } else if (fl & kfHelper) {
+              fl |= kfLHit;
+              mode = kDone;
+            } else {
+              finish(true);
+            }
+          }
+          if (ANY && exhausted) {
+            // helpers of owners that have just finished
+            const uint64_t busy = __ballot(mode != kIdle);
+            if ((fl & kfHelper) && mode != kIdle && !((busy >> own) & 1ull)) mode = kIdle;
+            if (mode == kIdle) helpers[tid] = 0u;
+          }
+        }
+      }
+      // ---- cheap work: pop with the reference's pop-time cull, expand ----
+      if (mode != kNode) continue;
+      if (cur == kNone) pop();
+      if (mode == kNode && !(cur & kLeafBit)) {
+        // one Node128: four child boxes tested axis by axis
+        static_assert(kWideKids == 4, "the expansion below is written for 4-wide nodes");
+        const float4* nd = nodes + (size_t)kWideNodeFloat4s * cur;
+        float4 a = nd[0], b = nd[3];
+        float n0, n1, n2, n3, f0, f1, f2, f3;
+        {
+          const float p0 = (a.x - o.x) * inv.x, q0 = (b.x - o.x) * inv.x;
+          const float p1 = (a.y - o.x) * inv.x, q1 = (b.y - o.x) * inv.x;
+          const float p2 = (a.z - o.x) * inv.x, q2 = (b.z - o.x) * inv.x;
+          const float p3 = (a.w - o.x) * inv.x, q3 = (b.w - o.x) * inv.x;
+          n0 = fminf(p0, q0), f0 = fmaxf(p0, q0);
+          n1 = fminf(p1, q1), f1 = fmaxf(p1, q1);
+          n2 = fminf(p2, q2), f2 = fmaxf(p2, q2);
+          n3 = fminf(p3, q3), f3 = fmaxf(p3, q3);
+        }
+        a = nd[1], b = nd[4];
+        {
+          const float p0 = (a.x - o.y) * inv.y, q0 = (b.x - o.y) * inv.y;
+          const float p1 = (a.y - o.y) * inv.y, q1 = (b.y - o.y) * inv.y;
+          const float p2 = (a.z - o.y) * inv.y, q2 = (b.z - o.y) * inv.y;
+          const float p3 = (a.w - o.y) * inv.y, q3 = (b.w - o.y) * inv.y;
+          n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
+          n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
+          n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
+          n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
+        }
+        a = nd[2], b = nd[5];
+        {
+          const float p0 = (a.x - o.z) * inv.z, q0 = (b.x - o.z) * inv.z;
+          const float p1 = (a.y - o.z) * inv.z, q1 = (b.y - o.z) * inv.z;
+          const float p2 = (a.z - o.z) * inv.z, q2 = (b.z - o.z) * inv.z;
+          const float p3 = (a.w - o.z) * inv.z, q3 = (b.w - o.z) * inv.z;
+          n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
+          n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
+          n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
+          n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
+        }
+        const uint4 r = *reinterpret_cast<const uint4*>(nd + 6);
+        // The slab test of each child: !(tNear > tFar || tFar < tMin), then
+        // the bound (the pop-time cull re-checks it against the best hit).
+        const bool k0 = r.x != kEmpty && !(n0 > f0 || f0 < tlow) && !(n0 > cullb);
+        const bool k1 = r.y != kEmpty && !(n1 > f1 || f1 < tlow) && !(n1 > cullb);
+        const bool k2 = r.z != kEmpty && !(n2 > f2 || f2 < tlow) && !(n2 > cullb);
+        const bool k3 = r.w != kEmpty && !(n3 > f3 || f3 < tlow) && !(n3 > cullb);
+        // Visit first: the nearest passing child (inside BLASes with
+        // near_first, lowest slot on equal distances), else the first passing
+        // slot, which is the reference's depth-first order.  The others are
+        // pushed so that they pop in slot order.
+        uint32_t first = k0 ? 0u : (k1 ? 1u : (k2 ? 2u : (k3 ? 3u : 4u)));
+        float bt = k0 ? n0 : (k1 ? n1 : (k2 ? n2 : n3));
+        const bool by_distance = (fl & kfLevel) ? near : (near_tlas && !(fl & kfRefOrder));
+        const bool c1 = k1 && by_distance && n1 < bt;
+        bt = c1 ? n1 : bt;
+        first = c1 ? 1u : first;
+        const bool c2 = k2 && by_distance && n2 < bt;
+        bt = c2 ? n2 : bt;
+        first = c2 ? 2u : first;
+        first = (k3 && by_distance && n3 < bt) ? 3u : first;
+        const bool u3 = k3 && first != 3u, u2 = k2 && first != 2u, u1 = k1 && first != 1u, u0 = k0 && first != 0u;
+        if (__builtin_expect(sp + 4u <= D, 1)) {
+          // without branches: each entry is written at the top, which moves
+          // past it only when its child is kept
+          st_ref[sp * B + tid] = r.w, st_tn[sp * B + tid] = n3;
+          sp += u3 ? 1u : 0u;
+          st_ref[sp * B + tid] = r.z, st_tn[sp * B + tid] = n2;
+          sp += u2 ? 1u : 0u;
+          st_ref[sp * B + tid] = r.y, st_tn[sp * B + tid] = n1;
+          sp += u1 ? 1u : 0u;
+          st_ref[sp * B + tid] = r.x, st_tn[sp * B + tid] = n0;
+          sp += u0 ? 1u : 0u;
+        } else {
+          for (uint32_t c = 4; c-- > 0;) {
+            const bool use = c == 3 ? u3 : (c == 2 ? u2 : (c == 1 ? u1 : u0));
+            if (!use) continue;
+            const uint32_t ref = c == 3 ? r.w : (c == 2 ? r.z : (c == 1 ? r.y : r.x));
+            const float tn = c == 3 ? n3 : (c == 2 ? n2 : (c == 1 ? n1 : n0));
+            if (sp < D) {
+              st_ref[sp * B + tid] = ref, st_tn[sp * B + tid] = tn;
+            } else if (sp < kWideStackCapacity) {
+              spill[(sp - D) * spill_stride + gtid] = (unsigned long long)ref | ((unsigned long long)f2u(tn) << 32);
+            } else {
+              atomicOr(p.error, 1u);  // the host's bound rules this out
+              continue;
+            }
+            ++sp;
+          }
+        }
+        cur = first == 0u ? r.x : (first == 1u ? r.y : (first == 2u ? r.z : (first == 3u ? r.w : kNone)));
+      }
+      // A leaf reached by the pop or the expansion becomes pending work.
+      if (mode == kNode && cur != kNone && (cur & kLeafBit)) {
+        mode = kLeaf;
+        if (!(fl & kfLevel)) {
+          slot = cur & 0x07FFFFFFu;
+          slot_end = slot + ((cur >> 27) & 15u);
+          cur = kNone;
+          mode = slot < slot_end ? kEnter : kNode;
+        }
+      }
+    }
+  }
+}
+
 __global__ void zero_u32_kernel(uint32_t* p, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0u;
@@ -936,64 +1690,52 @@ __global__ void fp32_selftest_kernel(const float* a, const float* b, float* q, f
 
 namespace vtk {
 
-template <bool ANY, bool COUNT, bool MULTI, bool W4>
+// The Node128 kernel when every scene has those trees (p.wide), else the
+// Node64 kernel.
+template <bool ANY, bool MULTI>
 static hipError_t launch_one(const TraceParams& p, uint32_t grid, hipStream_t s) {
-  hipLaunchKernelGGL((trace_kernel<ANY, COUNT, MULTI, W4, kTraceBlock, kLdsDepth>), dim3(grid),
-                     dim3(kTraceBlock), 0, s, p);
+  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, p.counter, 1u);
+  if (p.wide)
+    hipLaunchKernelGGL((wide_kernel<ANY, MULTI>), dim3(grid), dim3(kTraceBlock), 0, s, p);
+  else
+    hipLaunchKernelGGL((trace_kernel<ANY, false, MULTI, kTraceBlock, kLdsDepth>), dim3(grid), dim3(kTraceBlock), 0, s, p);
   return hipGetLastError();
 }
 
 hipError_t launch_trace_batch(const TraceParams& p, uint32_t grid, hipStream_t s) {
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, p.counter, 1u);
-  return p.wide ? launch_one<false, false, true, true>(p, grid, s)
-                             : launch_one<false, false, true, false>(p, grid, s);
+  return launch_one<false, true>(p, grid, s);
 }
 
 hipError_t launch_trace_batch_any(const TraceParams& p, uint32_t grid, hipStream_t s) {
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, p.counter, 1u);
-  return p.wide ? launch_one<true, false, true, true>(p, grid, s) : launch_one<true, false, true, false>(p, grid, s);
+  return launch_one<true, true>(p, grid, s);
 }
 
 hipError_t launch_trace(const TraceParams& p, bool any, bool count, uint32_t grid, hipStream_t s) {
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, p.counter, 1u);
-  if (count) return launch_one<false, true, false, false>(p, grid, s);
-  const bool w4 = p.wide != 0;
-  if (any) return w4 ? launch_one<true, false, false, true>(p, grid, s) : launch_one<true, false, false, false>(p, grid, s);
-  return w4 ? launch_one<false, false, false, true>(p, grid, s) : launch_one<false, false, false, false>(p, grid, s);
-}
-
-template <bool ANY, bool COUNT, bool MULTI, bool W4>
-static int occupancy_of() {
-  int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, trace_kernel<ANY, COUNT, MULTI, W4, kTraceBlock, kLdsDepth>,
-                                                   kTraceBlock, 0) != hipSuccess)
-    return -1;
-  return n;
-}
-
-static hipError_t min_occupancy(std::initializer_list<int> v, int* out) {
-  int m = 1 << 30;
-  for (int x : v) {
-    if (x < 0) return hipErrorInvalidValue;
-    m = x < m ? x : m;
+  if (count) {
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, p.counter, 1u);
+    hipLaunchKernelGGL((trace_kernel<false, true, false, kTraceBlock, kLdsDepth>), dim3(grid), dim3(kTraceBlock), 0, s, p);
+    return hipGetLastError();
   }
-  *out = m;
-  return hipSuccess;
+  return any ? launch_one<true, false>(p, grid, s) : launch_one<false, false>(p, grid, s);
 }
 
-hipError_t trace_occupancy_batch(int* blocks_per_cu) {
-  return min_occupancy({occupancy_of<false, false, true, false>(), occupancy_of<false, false, true, true>()},
-                       blocks_per_cu);
+// The smallest of the two kernels' resident blocks per CU.
+template <bool ANY, bool MULTI>
+static hipError_t occupancy_of(int* out) {
+  int a = 0, b = 0;
+  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      &a, trace_kernel<ANY, false, MULTI, kTraceBlock, kLdsDepth>, kTraceBlock, 0);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, wide_kernel<ANY, MULTI>, kTraceBlock, 0);
+  *out = a < b ? a : b;
+  return e;
 }
 
+hipError_t trace_occupancy_batch(int* blocks_per_cu) { return occupancy_of<false, true>(blocks_per_cu); }
+
+// The counting variant (measurement only) is left out: its extra blocks
+// simply start as others retire.
 hipError_t trace_occupancy(bool any, int* blocks_per_cu) {
-  if (any)
-    return min_occupancy({occupancy_of<true, false, false, false>(), occupancy_of<true, false, false, true>()},
-                         blocks_per_cu);
-  // The counting variant (measurement only) is left out: its extra blocks
-  // simply start as others retire.
-  return min_occupancy({occupancy_of<false, false, false, false>(), occupancy_of<false, false, false, true>()},
-                       blocks_per_cu);
+  return any ? occupancy_of<true, false>(blocks_per_cu) : occupancy_of<false, false>(blocks_per_cu);
 }
 
 hipError_t launch_zero(uint32_t* p, uint32_t n, hipStream_t s) {

@@ -60,3 +60,46 @@ def test_every_fill_matches_oracle(engine, make):
     finally:
         engine.set_hit_filter(0)
         engine.set_trace_tuning(8, 16, 2, 12)
+
+
+def _grazing(n, seed):
+    """A yawed box and rays that meet its faces at 1e-7 to 1e-2 rad, most near
+    the edges and vertices of the grid: hits shared by two triangles and
+    distances that the determinant hardly fixes."""
+    rng = np.random.default_rng(seed)
+    p, nn, i = W._merge([W._grid_quad(f[0], f[1], f[2], 20, 20, f[3])
+                         for f in W._box_faces((-0.33, 0.6, -0.28), (0.56, 1.2, 0.56), 15.0)])
+    sc = {"primitives": [W._mesh(p, nn, i, W.WHITE)], "scene_radius": 1.7}
+    tri = p[i[rng.integers(0, len(i), n)]]
+    b = rng.dirichlet([0.2, 0.2, 0.2], n)
+    normal = np.cross(tri[:, 1] - tri[:, 0], tri[:, 2] - tri[:, 0])
+    normal /= np.linalg.norm(normal, axis=1, keepdims=True)
+    d = rng.normal(size=(n, 3))
+    d -= normal * (d * normal).sum(1, keepdims=True)
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    d -= normal * (10 ** rng.uniform(-7, -2, n))[:, None]
+    rays = np.zeros(n, W.RAY_DTYPE)
+    rays["d"] = W._unit_f32(d.astype(np.float32))
+    rays["o"] = ((tri * b[:, :, None]).sum(1) - d * rng.uniform(0.01, 1.5, n)[:, None]).astype(np.float32)
+    rays["tmin"], rays["tmax"] = 1e-4, W.TMAX_INFINITY
+    return sc, rays
+
+
+def test_grazing_hits_do_not_depend_on_the_group(engine):
+    sc, rays = _grazing(40000, 4)
+    engine.set_scene(sc)
+    ps = O.PackedScene(O.pack_scene([dict(p, material_id=i) for i, p in enumerate(sc["primitives"])]))
+    try:
+        for near in (0, 1, 2):
+            engine.set_trace_tuning(8, 16, near, 12)
+            first = engine.trace_closest(rays)
+            if near == 0:  # the reference's order is exact, ties included
+                ref = O.trace_closest(ps, rays)
+                for k in FIELDS:
+                    assert np.array_equal(first[k].view(np.uint32), ref[k].view(np.uint32)), k
+            for seed in range(3):  # other neighbours in the wave, other lanes to help
+                order = np.random.default_rng(seed).permutation(rays.size)[: 40000 >> (2 * seed)]
+                assert np.array_equal(engine.trace_closest(rays[order]).view(np.uint8),
+                                      first[order].view(np.uint8)), (near, seed)
+    finally:
+        engine.set_trace_tuning(8, 16, 2, 12)

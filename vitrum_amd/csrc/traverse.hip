@@ -33,9 +33,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "traverse.h"
 #include "cwbvh.h"
+#include "fast_div.h"
 
 namespace vtk {
 
@@ -838,39 +840,18 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Division by a shared denominator
+// Operations with a shared denominator (fast_div.h)
 // ---------------------------------------------------------------------------
 
-// The correctly rounded quotient a / b from y, the refined reciprocal of b:
-// the residual-correction steps of the compiler's own expansion (two
-// remainders, each folded back with one fused multiply-add; Markstein, "IA-64
-// and Elementary Functions", 2000) without its operand scaling, which only
-// matters when a remainder or a quotient could leave the normal range.  The
-// callers check the operands with the two predicates below and divide
-// normally otherwise, so every quotient is the same bits.  Quotients that
-// share a denominator cost 6 instructions each instead of 11.
-__device__ __forceinline__ float recip_of(float b) {
-  const float y = __builtin_amdgcn_rcpf(b);
-  return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-__device__ __forceinline__ float div_by(float a, float b, float y) {
-  float q = a * y;
-  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-  return __builtin_amdgcn_div_fixupf(q, b, a);  // zeros, with their signs
-}
+using vtd::div_by;
+using vtd::div_den;
+using vtd::div_key;
+using vtd::kDivNum;
+using vtd::recip_of;
+
 __device__ __forceinline__ V3 div_by(V3 a, float b, float y) {
   return v3(div_by(a.x, b, y), div_by(a.y, b, y), div_by(a.z, b, y));
 }
-// |x| in [2^-40, 2^40]: a denominator.
-__device__ __forceinline__ bool div_den(float x) {
-  return (f2u(x) & 0x7FFFFFFFu) - 0x2B800000u <= 0x53800000u - 0x2B800000u;
-}
-// x zero or |x| >= 2^-60, as a key: numerators are safe when the smallest of
-// their keys is at least kDivNum (zero wraps to the largest key).  With a
-// denominator below 2^40 the quotient stays above 2^-100.
-constexpr uint32_t kDivNum = (0x21800000u << 1) - 1u;
-__device__ __forceinline__ uint32_t div_key(float x) { return (f2u(x) << 1) - 1u; }
 __device__ __forceinline__ uint32_t div_key(V3 a) { return min(min(div_key(a.x), div_key(a.y)), div_key(a.z)); }
 
 // xform_point, safe_normalize and safe_inv with the shared-denominator
@@ -1022,21 +1003,34 @@ __device__ __forceinline__ bool pair_test(V3 o, V3 dir, const WtRay& w, V3 a, V3
 // if it were its own.  The lane that entered the instance (the owner) waits
 // at the instance's exit until all its helpers are done and takes the
 // smallest (t, triangle) over them.  The group shares its best distance
-// through LDS.  A helped closest-hit walk visits boxes in another order, and
-// the order matters where two triangles are hit within the rounding of the
-// box tests: so a group culls against its best distance plus a margin
-// (2^-13 of the distance and the origin's magnitude, as for instances), and
-// when two hits come within that margin the owner walks the instance again
-// alone, in the usual order.  Without such a near-tie the nearest triangle is
-// never culled in any order, and it is the one that any order keeps.  Any-hit
-// answers do not depend on the order at all.
+// through LDS.  Any-hit answers do not depend on the order of a walk.  A
+// closest hit does in two rare cases, and a group that meets one of them
+// walks the instance again, its owner alone in the usual order:
+//  * Two hits within a margin of each other (2^-13 of the distance and the
+//    origin's magnitude, as between instances): which of them the pop-time
+//    cull lets through depends on the order.
+//  * A hit nearer than its own triangle's box by more than the margin.  The
+//    watertight distance is a weighted mean of the three vertices' depths
+//    along the ray's dominant axis; at a grazing angle (determinant near
+//    zero) the weights are inexact and it can fall anywhere between them,
+//    and whether such a triangle is tested depends on the order.
+// To see every such hit a group culls more cautiously than a lone lane:
+// against its best distance plus the margin, and by each box's near plane on
+// the dominant axis, which no distance of a triangle inside can undercut
+// (less 2^-20 of the slab for rounding); entries pushed before the lane
+// joined a group carry the usual entry distance and are culled by the bound
+// it had then, as the lone walk would have culled them.  Where neither case is
+// met, the nearest triangle is tested and kept in any order.
 //
 // Measured against the same walk without these three (trace_kernel over
-// Node128): 1,677,721 rays of the 1M-triangle scene 1.294 -> 0.944 ms;
+// Node128): 1,677,721 rays of the 1M-triangle scene 1.294 -> 1.033 ms;
 // 419,430 rays of the 32,768-triangle box, one launch after another on three
-// streams, 0.356 -> 0.157 ms and alone 0.99 -> 0.43 ms (its longest ray takes
+// streams, 0.356 -> 0.180 ms and alone 0.99 -> 0.45 ms (its longest ray takes
 // 322 steps, most rays under 60); a 256 x 256 path-traced frame of that box
-// (17 launches of at most 65,536 rays) 7.6 -> 3.1 ms.
+// (17 launches of at most 65,536 rays) 7.6 -> 2.9 ms.  Of this, the care that
+// makes a group's closest hit independent of its order costs 0.08 ms and
+// 0.025 ms of the first two; in one step loop for both phases instead of two
+// the first is 1.068 ms.
 constexpr uint32_t kIdle = 0, kNode = 1, kLeaf = 2, kEnter = 3, kExit = 4, kDone = 5;  // what a lane does next
 constexpr uint32_t kfHit = 1u;         // the record holds a hit
 constexpr uint32_t kfReject = 2u;      // ... on the back face of a single-sided material
@@ -1050,8 +1044,8 @@ constexpr uint32_t kfLFront = 256u;
 constexpr uint32_t kfLSingle = 512u;
 constexpr uint32_t kfSplit = 1024u;    // in a group: an owner with helpers, or a helper
 constexpr uint32_t kfHelper = 2048u;
-constexpr uint32_t kfTie = 4096u;      // two hits of the group came within the margin
-constexpr uint32_t kfAlone = 8192u;    // no helpers in this instance (walked again after a near-tie)
+constexpr uint32_t kfTie = 4096u;      // the group met a hit whose fate depends on the order
+constexpr uint32_t kfAlone = 8192u;    // no helpers in this instance (walked again because of kfTie)
 constexpr uint32_t kfLocal = kfLevel | kfMirror | kfWt | kfLHit | kfLFront | kfLSingle | kfSplit | kfTie;
 constexpr uint32_t kHelpSteps = 4;     // steps between two rounds of taking work
 
@@ -1095,9 +1089,11 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
   // Local: direction, watertight set-up, best hit, the bound it entered with.
   V3 ld{}, lpos{};
   WtRay lw{};
-  float lbest = 0, lcap = 0, lu = 0, lv = 0;
+  float lbest = 0, lcap = 0, cull0 = 0, lu = 0, lv = 0;
   uint32_t lprim = 0, slot = 0, slot_end = 0, own = lane;
-  uint32_t cur = kNone, sp = 0, base = 0, tsp = 0;  // stack: next entry, the level's first, the TLAS part's end
+  // Stack: next entry, the level's first, the TLAS part's end, and the end of
+  // the entries pushed before joining a group (culled by `cull0`).
+  uint32_t cur = kNone, sp = 0, base = 0, tsp = 0, mark = 0;
 
   auto scene_of = [&]() -> const DeviceScene& { return MULTI ? p.scenes[sid] : p.scene; };
   auto margin = [&](float t) { return (t + max(fabs_(o.x), max(fabs_(o.y), fabs_(o.z)))) * 0x1p-13f; };
@@ -1137,11 +1133,14 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
     mode = kNode;
   };
   // A lane's subtree or interval is done: the next entry that its bound keeps.
-  auto pop = [&]() {
+  auto pop = [&](auto helping) {
+    constexpr bool GROUP = !ANY && decltype(helping)::value;
     for (;;) {
       if (sp > base) {
         const uint2 e = stk_load(--sp);
-        if (u2f(e.y) > cullb) continue;
+        const bool before = GROUP && (fl & kfSplit) && sp < mark;
+        if (GROUP) mark = before ? sp : mark;
+        if (u2f(e.y) > (before ? cull0 : cullb)) continue;
         cur = e.x;
         return;
       }
@@ -1177,115 +1176,122 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
     }
   };
 
-  // The first fill is static, later ones go through the shared counter (see
-  // trace_kernel); `exhausted`: no more rays for this wave.
-  bool exhausted = false, first_fill = true;
-  for (;;) {
-    const uint64_t idle = __ballot(mode == kIdle);
-    const uint32_t n_idle = (uint32_t)__popcll(idle);
-    if (!exhausted) {
-      if (n_idle >= p.refill_min || n_idle == 64u) {
-        const uint32_t take = min(n_idle, take_cap);
-        uint32_t first = wave_id * take_cap;
-        if (!first_fill) {
-          if (lane == 0) first = static_end + atomicAdd(p.counter, take);
-          first = (uint32_t)__shfl((int)first, 0);
+  // One step of a lane with an interior node: its four children.
+  auto expand = [&](auto helping) {
+    constexpr bool GROUP = !ANY && decltype(helping)::value;
+    // one Node128: four child boxes tested axis by axis
+    static_assert(kWideKids == 4, "the expansion below is written for 4-wide nodes");
+    const float4* nd = nodes + (size_t)kWideNodeFloat4s * cur;
+    float4 a = nd[0], b = nd[3];
+    float n0, n1, n2, n3, f0, f1, f2, f3;
+    {
+      const float p0 = (a.x - o.x) * inv.x, q0 = (b.x - o.x) * inv.x;
+      const float p1 = (a.y - o.x) * inv.x, q1 = (b.y - o.x) * inv.x;
+      const float p2 = (a.z - o.x) * inv.x, q2 = (b.z - o.x) * inv.x;
+      const float p3 = (a.w - o.x) * inv.x, q3 = (b.w - o.x) * inv.x;
+      n0 = fminf(p0, q0), f0 = fmaxf(p0, q0);
+      n1 = fminf(p1, q1), f1 = fmaxf(p1, q1);
+      n2 = fminf(p2, q2), f2 = fmaxf(p2, q2);
+      n3 = fminf(p3, q3), f3 = fmaxf(p3, q3);
+    }
+    a = nd[1], b = nd[4];
+    {
+      const float p0 = (a.x - o.y) * inv.y, q0 = (b.x - o.y) * inv.y;
+      const float p1 = (a.y - o.y) * inv.y, q1 = (b.y - o.y) * inv.y;
+      const float p2 = (a.z - o.y) * inv.y, q2 = (b.z - o.y) * inv.y;
+      const float p3 = (a.w - o.y) * inv.y, q3 = (b.w - o.y) * inv.y;
+      n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
+      n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
+      n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
+      n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
+    }
+    a = nd[2], b = nd[5];
+    {
+      const float p0 = (a.x - o.z) * inv.z, q0 = (b.x - o.z) * inv.z;
+      const float p1 = (a.y - o.z) * inv.z, q1 = (b.y - o.z) * inv.z;
+      const float p2 = (a.z - o.z) * inv.z, q2 = (b.z - o.z) * inv.z;
+      const float p3 = (a.w - o.z) * inv.z, q3 = (b.w - o.z) * inv.z;
+      n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
+      n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
+      n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
+      n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
+    }
+    const uint4 r = *reinterpret_cast<const uint4*>(nd + 6);
+    // What the bound culls and the stack keeps: the entry distance, in a
+    // group the near plane on the dominant axis.
+    float g0 = n0, g1 = n1, g2 = n2, g3 = n3;
+    if (GROUP && (fl & kfSplit)) {
+      const int kz = (int)min((lw.perm >> 4) & 3u, 2u);
+      const float4 lo_k = nd[kz], hi_k = nd[3 + kz];
+      const float ok = sel3(kz, o.x, o.y, o.z), ik = sel3(kz, inv.x, inv.y, inv.z);
+      auto near_plane = [&](float mn, float mx) {
+        const float p = (mn - ok) * ik, q = (mx - ok) * ik;
+        return fminf(p, q) - fmaxf(fabs_(p), fabs_(q)) * 0x1p-20f;
+      };
+      g0 = near_plane(lo_k.x, hi_k.x);
+      g1 = near_plane(lo_k.y, hi_k.y);
+      g2 = near_plane(lo_k.z, hi_k.z);
+      g3 = near_plane(lo_k.w, hi_k.w);
+    }
+    // The slab test of each child: !(tNear > tFar || tFar < tMin), then
+    // the bound (the pop-time cull re-checks it against the best hit).
+    const bool k0 = r.x != kEmpty && !(n0 > f0 || f0 < tlow) && !(g0 > cullb);
+    const bool k1 = r.y != kEmpty && !(n1 > f1 || f1 < tlow) && !(g1 > cullb);
+    const bool k2 = r.z != kEmpty && !(n2 > f2 || f2 < tlow) && !(g2 > cullb);
+    const bool k3 = r.w != kEmpty && !(n3 > f3 || f3 < tlow) && !(g3 > cullb);
+    // Visit first: the nearest passing child (inside BLASes with
+    // near_first, lowest slot on equal distances), else the first passing
+    // slot, which is the reference's depth-first order.  The others are
+    // pushed so that they pop in slot order.
+    uint32_t first = k0 ? 0u : (k1 ? 1u : (k2 ? 2u : (k3 ? 3u : 4u)));
+    float bt = k0 ? n0 : (k1 ? n1 : (k2 ? n2 : n3));
+    const bool by_distance = (fl & kfLevel) ? near : (near_tlas && !(fl & kfRefOrder));
+    const bool c1 = k1 && by_distance && n1 < bt;
+    bt = c1 ? n1 : bt;
+    first = c1 ? 1u : first;
+    const bool c2 = k2 && by_distance && n2 < bt;
+    bt = c2 ? n2 : bt;
+    first = c2 ? 2u : first;
+    first = (k3 && by_distance && n3 < bt) ? 3u : first;
+    const bool u3 = k3 && first != 3u, u2 = k2 && first != 2u, u1 = k1 && first != 1u, u0 = k0 && first != 0u;
+    if (__builtin_expect(sp + 4u <= D, 1)) {
+      // without branches: each entry is written at the top, which moves
+      // past it only when its child is kept
+      st_ref[sp * B + tid] = r.w, st_tn[sp * B + tid] = g3;
+      sp += u3 ? 1u : 0u;
+      st_ref[sp * B + tid] = r.z, st_tn[sp * B + tid] = g2;
+      sp += u2 ? 1u : 0u;
+      st_ref[sp * B + tid] = r.y, st_tn[sp * B + tid] = g1;
+      sp += u1 ? 1u : 0u;
+      st_ref[sp * B + tid] = r.x, st_tn[sp * B + tid] = g0;
+      sp += u0 ? 1u : 0u;
+    } else {
+      for (uint32_t c = 4; c-- > 0;) {
+        const bool use = c == 3 ? u3 : (c == 2 ? u2 : (c == 1 ? u1 : u0));
+        if (!use) continue;
+        const uint32_t ref = c == 3 ? r.w : (c == 2 ? r.z : (c == 1 ? r.y : r.x));
+        const float tn = c == 3 ? g3 : (c == 2 ? g2 : (c == 1 ? g1 : g0));
+        if (sp < D) {
+          st_ref[sp * B + tid] = ref, st_tn[sp * B + tid] = tn;
+        } else if (sp < kWideStackCapacity) {
+          spill[(sp - D) * spill_stride + gtid] = (unsigned long long)ref | ((unsigned long long)f2u(tn) << 32);
+        } else {
+          atomicOr(p.error, 1u);  // the host's bound rules this out
+          continue;
         }
-        first_fill = false;
-        exhausted = first + take >= n_rays;
-        const uint32_t rank = (uint32_t)__popcll(idle & lane_below), idx = first + rank;
-        if (mode == kIdle && rank < take && idx < n_rays) {
-          ray_idx = idx;
-          if (MULTI) {
-            uint32_t lo_s = 0, hi_s = p.scene_count;
-            while (lo_s + 1u < hi_s) {
-              const uint32_t mid = (lo_s + hi_s) >> 1;
-              if (p.scene_offsets[mid] <= idx) lo_s = mid; else hi_s = mid;
-            }
-            sid = lo_s;
-          }
-          const float4 a = p.rays[2 * (size_t)idx], b = p.rays[2 * (size_t)idx + 1];
-          const DeviceScene& S = scene_of();
-          nodes = S.tlas4_nodes;
-          o = v3(a.x, a.y, a.z);
-          inv = safe_inv3(v3(b.x, b.y, b.z));
-          wlow = a.w;
-          best = b.w;
-          fl = 0;
-          own = lane;
-          restart();
-          if (S.tlas_node_count == 0u) finish(false);  // no TLAS: fail closed
-        }
-      }
-    } else if (idle != 0ull && n_idle != 64u) {
-      // ---- share the groups' bounds, then hand out work ----
-      if (mode == kIdle) fl = 0;
-      if (!ANY && (fl & kfSplit)) {
-        if (fl & kfLHit) atomicMin(&group_best[wbase + own], f2u(lbest));  // t > 0: ordered as integers
-      }
-      wave_sync();
-      if (!ANY && (fl & kfSplit)) {
-        const float g = u2f(group_best[wbase + own]);
-        cullb = fminf(cullb, g + margin(g));
-      }
-      const bool donor = (fl & (kfLevel | kfAlone)) == kfLevel && (mode == kNode || mode == kLeaf) && sp > base && base < D;
-      const uint64_t donors = __ballot(donor);
-      if (donors != 0ull) {
-        // The r-th idle lane takes entry r / n_donors of donor r % n_donors.
-        const uint32_t n_don = (uint32_t)__popcll(donors), rank_d = (uint32_t)__popcll(donors & lane_below);
-        const uint32_t avail = donor ? min(sp, D) - base : 0u;
-        if (donor) table[wbase + rank_d] = lane;
-        wave_sync();
-        const uint32_t r = (uint32_t)__popcll(idle & lane_below), k = r / n_don;
-        const int d = mode == kIdle ? (int)table[wbase + (r - k * n_don)] : (int)lane;
-        wave_sync();
-        const uint32_t d_avail = (uint32_t)__shfl((int)avail, d);
-        const bool got = mode == kIdle && k < d_avail;
-        const uint32_t at = (uint32_t)__shfl((int)base, d) + k;
-        const uint32_t d_own = (uint32_t)__shfl((int)own, d), d_fl = (uint32_t)__shfl((int)fl, d);
-        const V3 d_o = v3(__shfl(o.x, d), __shfl(o.y, d), __shfl(o.z, d));
-        const V3 d_inv = v3(__shfl(inv.x, d), __shfl(inv.y, d), __shfl(inv.z, d));
-        const V3 d_ld = v3(__shfl(ld.x, d), __shfl(ld.y, d), __shfl(ld.z, d));
-        const float d_low = __shfl(tlow, d), d_cull = __shfl(cullb, d), d_cap = __shfl(lcap, d);
-        const uint64_t d_nodes = (uint64_t)(uintptr_t)nodes;
-        const uint32_t d_nlo = (uint32_t)__shfl((int)(uint32_t)d_nodes, d);
-        const uint32_t d_nhi = (uint32_t)__shfl((int)(uint32_t)(d_nodes >> 32), d);
-        const uint32_t d_sid = MULTI ? (uint32_t)__shfl((int)sid, d) : 0u;
-        if (donor) {
-          const uint32_t share = n_idle > rank_d ? (n_idle - rank_d - 1u) / n_don + 1u : 0u;
-          base += min(avail, share);
-          if (share != 0u && !(fl & kfSplit)) {
-            fl |= kfSplit;
-            if (!ANY) group_best[tid] = (fl & kfLHit) ? f2u(lbest) : 0x7F7FFFFFu;
-          }
-        }
-        wave_sync();
-        if (got) {
-          const uint32_t ref = st_ref[at * B + wbase + (uint32_t)d];
-          const float tn = st_tn[at * B + wbase + (uint32_t)d];
-          own = d_own;
-          o = d_o;
-          inv = d_inv;
-          ld = d_ld;
-          tlow = d_low;
-          cullb = d_cull;
-          lcap = d_cap;
-          nodes = reinterpret_cast<const float4*>((uintptr_t)(((uint64_t)d_nhi << 32) | d_nlo));
-          sid = d_sid;
-          fl = kfHelper | kfSplit | kfLevel | (d_fl & kfMirror);
-          lbest = d_cap;
-          sp = base = tsp = 0;
-          cur = tn > cullb ? kNone : ref;
-          mode = (cur != kNone && (cur & kLeafBit)) ? kLeaf : kNode;
-          atomicAdd(&helpers[wbase + own], 1u);
-        }
+        ++sp;
       }
     }
-    if (!__any(mode != kIdle)) break;
+    cur = first == 0u ? r.x : (first == 1u ? r.y : (first == 2u ? r.z : (first == 3u ? r.w : kNone)));
+  };
 
-    const uint32_t n_steps = exhausted ? kHelpSteps : p.steps;
+  // `n_steps` steps of the wave: deferred work, then a node each.  Built twice:
+  // without anything about groups for the time the wave still fetches rays,
+  // and with it (`helping`) for the time after.
+  auto run = [&](auto helping, uint32_t n_steps) {
+    constexpr bool HELP = decltype(helping)::value, GROUP = !ANY && HELP;
     for (uint32_t step = 0; step < n_steps; ++step) {
-      if (exhausted) {
+      if (HELP) {
         // ---- helpers that are done ----
         uint64_t done = __ballot(mode == kDone);
         if (done) {
@@ -1340,11 +1346,11 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
       const uint32_t dm = min(p.defer_min, ((uint32_t)__popcll(m_pend | m_cheap) + 1u) >> 1);
       if (m_cheap == 0ull || (uint32_t)__popcll(m_pend) >= dm) {
         const bool all = m_cheap == 0ull;
-        const bool at_exit = mode == kExit && !((fl & kfSplit) && helpers[tid] != 0u);
+        const bool at_exit = mode == kExit && !(HELP && (fl & kfSplit) && helpers[tid] != 0u);
         const uint64_t m_exit = __ballot(at_exit);
         const uint64_t m_enter = __ballot(mode == kEnter);
         const uint64_t m_leaf = __ballot(mode == kLeaf);
-        if (all && (m_exit | m_enter | m_leaf) == 0ull) {
+        if (HELP && all && (m_exit | m_enter | m_leaf) == 0ull) {
           // Only owners that wait, and no helper to wait for: cannot happen.
           // Report it and end the wave rather than wait for ever.
           if (lane == 0) atomicOr(p.error, 2u);
@@ -1356,8 +1362,11 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
           cur = kNone;
           sp = tsp;
           base = 0;
-          if (!ANY && (fl & kfTie)) {
-            // a near-tie inside the group: this instance again, alone
+          // (a hit within the margin of the bound the walk entered with is
+          // the same kind of tie)
+          if (GROUP && (fl & kfSplit) && (fl & kfLHit) && lcap - lbest <= margin(lbest)) fl |= kfTie;
+          if (GROUP && (fl & kfTie)) {
+            // this instance again, alone
             fl = (fl & ~kfLocal) | kfAlone;
             mode = kEnter;
           } else {
@@ -1477,7 +1486,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
             const float w_low = __shfl(tlow, ol);
             // An owner or helper accepts up to its cull bound (its best plus
             // the margin); otherwise hits below the best, or at it.
-            const float w_hi = __shfl((fl & kfSplit) ? cullb : lbest, ol);
+            const float w_hi = __shfl(GROUP && (fl & kfSplit) ? cullb : lbest, ol);
             const uint32_t w_fl = (uint32_t)__shfl((int)fl, ol);
             const float4* otris = p.scene.tris;
             if (MULTI) otris = p.scenes[(uint32_t)__shfl((int)sid, ol)].tris;
@@ -1492,13 +1501,29 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
               const float4 w0 = tr[0], w1 = tr[1], w2 = tr[2];
               single = w2.y;
               hit = pair_test(wo, wd, ww, v3(w0.x, w0.y, w0.z), v3(w0.w, w1.x, w1.y), v3(w1.z, w1.w, w2.x), w_low, w_hi,
-                              near && (w_fl & (kfLHit | kfSplit)) == kfLHit, h);
+                              near && (w_fl & (GROUP ? kfLHit | kfSplit : kfLHit)) == kfLHit, h);
               // Any hit through the path tracer's wrappers: a back face of a
               // single-sided material does not block.
               if (ANY && hit && p.sided && h.front == ((w_fl & kfMirror) != 0u) && single > 0.5f) hit = false;
             }
             const uint64_t hits = __ballot(hit);
             if (hits == 0ull) continue;
+            uint64_t early = 0ull;  // hits nearer than their own triangle's box
+            if (GROUP && __any((fl & kfSplit) != 0u)) {
+              const V3 wi = v3(__shfl(inv.x, ol), __shfl(inv.y, ol), __shfl(inv.z, ol));
+              bool e = false;
+              if (hit) {
+                const float4* tr = otris + 3 * (size_t)tri;
+                const float4 w0 = tr[0], w1 = tr[1], w2 = tr[2];
+                float tn;
+                (void)slab(wo, wi, fminf(w0.x, fminf(w0.w, w1.z)), fminf(w0.y, fminf(w1.x, w1.w)),
+                           fminf(w0.z, fminf(w1.y, w2.x)), fmaxf(w0.x, fmaxf(w0.w, w1.z)),
+                           fmaxf(w0.y, fmaxf(w1.x, w1.w)), fmaxf(w0.z, fmaxf(w1.y, w2.x)), w_low, tn);
+                const float m = (h.t + max(fabs_(wo.x), max(fabs_(wo.y), fabs_(wo.z)))) * 0x1p-13f;
+                e = !(h.t >= tn - m);
+              }
+              early = __ballot(e);
+            }
             // Each ray's run of lanes in this round: [lo, hi).
             const uint32_t lo = min(max(excl, first) - first, 64u), hi = min(max(excl + cnt, first) - first, 64u);
             const uint64_t run = (hi > lo) ? ((~0ull >> (64u - (hi - lo))) << lo) & hits : 0ull;
@@ -1522,9 +1547,9 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
             const V3 rp = v3(__shfl(h.point.x, (int)rl), __shfl(h.point.y, (int)rl), __shfl(h.point.z, (int)rl));
             const uint32_t rb = (uint32_t)__shfl((int)bits, (int)rl);
             if (run != 0ull) {
-              if (fl & kfSplit) {
+              if (GROUP && (fl & kfSplit)) {
                 // two hits in one leaf, or one within the margin of the best
-                if ((run & (run - 1ull)) != 0ull) fl |= kfTie;
+                if ((run & (run - 1ull)) != 0ull || (run & early) != 0ull) fl |= kfTie;
                 if ((fl & kfLHit) && fabs_(rt - lbest) <= margin(fminf(rt, lbest))) fl |= kfTie;
               }
               if (!(fl & kfLHit) || rt < lbest || (rt == lbest && ri < lprim)) {
@@ -1534,22 +1559,20 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
                 lu = ru;
                 lv = rv;
                 lpos = rp;
-                cullb = (fl & kfSplit) ? fminf(cullb, fminf(lcap, rt + margin(rt))) : rt;
+                cullb = GROUP && (fl & kfSplit) ? fminf(cullb, fminf(lcap, rt + margin(rt))) : rt;
               }
             }
           }
           if (ANY && occl) {
             // A group's lanes end together, at the owner.
-            if (!(fl & kfSplit)) {
-              finish(true);
-            } else if (fl & kfHelper) {
+            if (HELP && (fl & kfHelper)) {
               fl |= kfLHit;
               mode = kDone;
             } else {
               finish(true);
             }
           }
-          if (ANY && exhausted) {
+          if (ANY && HELP) {
             // helpers of owners that have just finished
             const uint64_t busy = __ballot(mode != kIdle);
             if ((fl & kfHelper) && mode != kIdle && !((busy >> own) & 1ull)) mode = kIdle;
@@ -1559,97 +1582,8 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
       }
       // ---- cheap work: pop with the reference's pop-time cull, expand ----
       if (mode != kNode) continue;
-      if (cur == kNone) pop();
-      if (mode == kNode && !(cur & kLeafBit)) {
-        // one Node128: four child boxes tested axis by axis
-        static_assert(kWideKids == 4, "the expansion below is written for 4-wide nodes");
-        const float4* nd = nodes + (size_t)kWideNodeFloat4s * cur;
-        float4 a = nd[0], b = nd[3];
-        float n0, n1, n2, n3, f0, f1, f2, f3;
-        {
-          const float p0 = (a.x - o.x) * inv.x, q0 = (b.x - o.x) * inv.x;
-          const float p1 = (a.y - o.x) * inv.x, q1 = (b.y - o.x) * inv.x;
-          const float p2 = (a.z - o.x) * inv.x, q2 = (b.z - o.x) * inv.x;
-          const float p3 = (a.w - o.x) * inv.x, q3 = (b.w - o.x) * inv.x;
-          n0 = fminf(p0, q0), f0 = fmaxf(p0, q0);
-          n1 = fminf(p1, q1), f1 = fmaxf(p1, q1);
-          n2 = fminf(p2, q2), f2 = fmaxf(p2, q2);
-          n3 = fminf(p3, q3), f3 = fmaxf(p3, q3);
-        }
-        a = nd[1], b = nd[4];
-        {
-          const float p0 = (a.x - o.y) * inv.y, q0 = (b.x - o.y) * inv.y;
-          const float p1 = (a.y - o.y) * inv.y, q1 = (b.y - o.y) * inv.y;
-          const float p2 = (a.z - o.y) * inv.y, q2 = (b.z - o.y) * inv.y;
-          const float p3 = (a.w - o.y) * inv.y, q3 = (b.w - o.y) * inv.y;
-          n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
-          n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
-          n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
-          n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
-        }
-        a = nd[2], b = nd[5];
-        {
-          const float p0 = (a.x - o.z) * inv.z, q0 = (b.x - o.z) * inv.z;
-          const float p1 = (a.y - o.z) * inv.z, q1 = (b.y - o.z) * inv.z;
-          const float p2 = (a.z - o.z) * inv.z, q2 = (b.z - o.z) * inv.z;
-          const float p3 = (a.w - o.z) * inv.z, q3 = (b.w - o.z) * inv.z;
-          n0 = fmaxf(n0, fminf(p0, q0)), f0 = fminf(f0, fmaxf(p0, q0));
-          n1 = fmaxf(n1, fminf(p1, q1)), f1 = fminf(f1, fmaxf(p1, q1));
-          n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
-          n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
-        }
-        const uint4 r = *reinterpret_cast<const uint4*>(nd + 6);
-        // The slab test of each child: !(tNear > tFar || tFar < tMin), then
-        // the bound (the pop-time cull re-checks it against the best hit).
-        const bool k0 = r.x != kEmpty && !(n0 > f0 || f0 < tlow) && !(n0 > cullb);
-        const bool k1 = r.y != kEmpty && !(n1 > f1 || f1 < tlow) && !(n1 > cullb);
-        const bool k2 = r.z != kEmpty && !(n2 > f2 || f2 < tlow) && !(n2 > cullb);
-        const bool k3 = r.w != kEmpty && !(n3 > f3 || f3 < tlow) && !(n3 > cullb);
-        // Visit first: the nearest passing child (inside BLASes with
-        // near_first, lowest slot on equal distances), else the first passing
-        // slot, which is the reference's depth-first order.  The others are
-        // pushed so that they pop in slot order.
-        uint32_t first = k0 ? 0u : (k1 ? 1u : (k2 ? 2u : (k3 ? 3u : 4u)));
-        float bt = k0 ? n0 : (k1 ? n1 : (k2 ? n2 : n3));
-        const bool by_distance = (fl & kfLevel) ? near : (near_tlas && !(fl & kfRefOrder));
-        const bool c1 = k1 && by_distance && n1 < bt;
-        bt = c1 ? n1 : bt;
-        first = c1 ? 1u : first;
-        const bool c2 = k2 && by_distance && n2 < bt;
-        bt = c2 ? n2 : bt;
-        first = c2 ? 2u : first;
-        first = (k3 && by_distance && n3 < bt) ? 3u : first;
-        const bool u3 = k3 && first != 3u, u2 = k2 && first != 2u, u1 = k1 && first != 1u, u0 = k0 && first != 0u;
-        if (__builtin_expect(sp + 4u <= D, 1)) {
-          // without branches: each entry is written at the top, which moves
-          // past it only when its child is kept
-          st_ref[sp * B + tid] = r.w, st_tn[sp * B + tid] = n3;
-          sp += u3 ? 1u : 0u;
-          st_ref[sp * B + tid] = r.z, st_tn[sp * B + tid] = n2;
-          sp += u2 ? 1u : 0u;
-          st_ref[sp * B + tid] = r.y, st_tn[sp * B + tid] = n1;
-          sp += u1 ? 1u : 0u;
-          st_ref[sp * B + tid] = r.x, st_tn[sp * B + tid] = n0;
-          sp += u0 ? 1u : 0u;
-        } else {
-          for (uint32_t c = 4; c-- > 0;) {
-            const bool use = c == 3 ? u3 : (c == 2 ? u2 : (c == 1 ? u1 : u0));
-            if (!use) continue;
-            const uint32_t ref = c == 3 ? r.w : (c == 2 ? r.z : (c == 1 ? r.y : r.x));
-            const float tn = c == 3 ? n3 : (c == 2 ? n2 : (c == 1 ? n1 : n0));
-            if (sp < D) {
-              st_ref[sp * B + tid] = ref, st_tn[sp * B + tid] = tn;
-            } else if (sp < kWideStackCapacity) {
-              spill[(sp - D) * spill_stride + gtid] = (unsigned long long)ref | ((unsigned long long)f2u(tn) << 32);
-            } else {
-              atomicOr(p.error, 1u);  // the host's bound rules this out
-              continue;
-            }
-            ++sp;
-          }
-        }
-        cur = first == 0u ? r.x : (first == 1u ? r.y : (first == 2u ? r.z : (first == 3u ? r.w : kNone)));
-      }
+      if (cur == kNone) pop(helping);
+      if (mode == kNode && !(cur & kLeafBit)) expand(helping);
       // A leaf reached by the pop or the expansion becomes pending work.
       if (mode == kNode && cur != kNone && (cur & kLeafBit)) {
         mode = kLeaf;
@@ -1661,6 +1595,132 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         }
       }
     }
+  };
+
+  // The first fill is static, later ones go through the shared counter (see
+  // trace_kernel); `exhausted`: no more rays for this wave.
+  bool exhausted = false, first_fill = true;
+  for (;;) {
+    const uint64_t idle = __ballot(mode == kIdle);
+    const uint32_t n_idle = (uint32_t)__popcll(idle);
+    if (!exhausted) {
+      if (n_idle >= p.refill_min || n_idle == 64u) {
+        const uint32_t take = min(n_idle, take_cap);
+        uint32_t first = wave_id * take_cap;
+        if (!first_fill) {
+          if (lane == 0) first = static_end + atomicAdd(p.counter, take);
+          first = (uint32_t)__shfl((int)first, 0);
+        }
+        first_fill = false;
+        exhausted = first + take >= n_rays;
+        const uint32_t rank = (uint32_t)__popcll(idle & lane_below), idx = first + rank;
+        if (mode == kIdle && rank < take && idx < n_rays) {
+          ray_idx = idx;
+          if (MULTI) {
+            uint32_t lo_s = 0, hi_s = p.scene_count;
+            while (lo_s + 1u < hi_s) {
+              const uint32_t mid = (lo_s + hi_s) >> 1;
+              if (p.scene_offsets[mid] <= idx) lo_s = mid; else hi_s = mid;
+            }
+            sid = lo_s;
+          }
+          const float4 a = p.rays[2 * (size_t)idx], b = p.rays[2 * (size_t)idx + 1];
+          const DeviceScene& S = scene_of();
+          nodes = S.tlas4_nodes;
+          o = v3(a.x, a.y, a.z);
+          inv = safe_inv3(v3(b.x, b.y, b.z));
+          wlow = a.w;
+          best = b.w;
+          fl = 0;
+          own = lane;
+          restart();
+          if (S.tlas_node_count == 0u) finish(false);  // no TLAS: fail closed
+        }
+      }
+    } else if (idle != 0ull && n_idle != 64u) {
+      // ---- share the groups' bounds, then hand out work ----
+      if (mode == kIdle) fl = 0;
+      if (!ANY && (fl & kfSplit)) {
+        if (fl & kfLHit) atomicMin(&group_best[wbase + own], f2u(lbest));  // t > 0: ordered as integers
+      }
+      wave_sync();
+      if (!ANY && (fl & kfSplit)) {
+        const float g = u2f(group_best[wbase + own]);
+        cullb = fminf(cullb, g + margin(g));
+      }
+      const bool donor = (fl & (kfLevel | kfAlone)) == kfLevel && (mode == kNode || mode == kLeaf) && sp > base && base < D;
+      const uint64_t donors = __ballot(donor);
+      if (donors != 0ull) {
+        // The r-th idle lane takes entry r / n_donors of donor r % n_donors.
+        const uint32_t n_don = (uint32_t)__popcll(donors), rank_d = (uint32_t)__popcll(donors & lane_below);
+        const uint32_t share = donor && n_idle > rank_d ? (n_idle - rank_d - 1u) / n_don + 1u : 0u;
+        if (donor && !(fl & kfWt)) {
+          lw = wt_setup(ld);
+          fl |= kfWt;
+        }
+        if (share != 0u && !(fl & kfSplit)) {
+          fl |= kfSplit;
+          mark = sp;
+          cull0 = cullb;
+          if (!ANY) group_best[tid] = (fl & kfLHit) ? f2u(lbest) : 0x7F7FFFFFu;
+          if (!ANY && (fl & kfLHit)) cullb = fminf(lcap, lbest + margin(lbest));
+        }
+        const uint32_t avail = donor ? min(sp, D) - base : 0u;
+        if (donor) table[wbase + rank_d] = lane;
+        wave_sync();
+        const uint32_t r = (uint32_t)__popcll(idle & lane_below), k = r / n_don;
+        const int d = mode == kIdle ? (int)table[wbase + (r - k * n_don)] : (int)lane;
+        wave_sync();
+        const uint32_t d_avail = (uint32_t)__shfl((int)avail, d);
+        const bool got = mode == kIdle && k < d_avail;
+        const uint32_t at = (uint32_t)__shfl((int)base, d) + k;
+        const uint32_t d_own = (uint32_t)__shfl((int)own, d), d_fl = (uint32_t)__shfl((int)fl, d);
+        const V3 d_o = v3(__shfl(o.x, d), __shfl(o.y, d), __shfl(o.z, d));
+        const V3 d_inv = v3(__shfl(inv.x, d), __shfl(inv.y, d), __shfl(inv.z, d));
+        const V3 d_ld = v3(__shfl(ld.x, d), __shfl(ld.y, d), __shfl(ld.z, d));
+        const float d_low = __shfl(tlow, d), d_cull = __shfl(cullb, d), d_cap = __shfl(lcap, d);
+        const float d_cull0 = __shfl(cull0, d);
+        const uint32_t d_mark = (uint32_t)__shfl((int)mark, d);
+        const uint64_t d_nodes = (uint64_t)(uintptr_t)nodes;
+        const uint32_t d_nlo = (uint32_t)__shfl((int)(uint32_t)d_nodes, d);
+        const uint32_t d_nhi = (uint32_t)__shfl((int)(uint32_t)(d_nodes >> 32), d);
+        const uint32_t d_sid = MULTI ? (uint32_t)__shfl((int)sid, d) : 0u;
+        WtRay d_lw;
+        d_lw.ds = __shfl(lw.ds, d);
+        d_lw.sx = __shfl(lw.sx, d);
+        d_lw.sy = __shfl(lw.sy, d);
+        d_lw.sz = __shfl(lw.sz, d);
+        d_lw.perm = (uint32_t)__shfl((int)lw.perm, d);
+        if (donor) base += min(avail, share);
+        wave_sync();
+        if (got) {
+          const uint32_t ref = st_ref[at * B + wbase + (uint32_t)d];
+          const float tn = st_tn[at * B + wbase + (uint32_t)d];
+          own = d_own;
+          lw = d_lw;
+          o = d_o;
+          inv = d_inv;
+          ld = d_ld;
+          tlow = d_low;
+          cullb = d_cull;
+          lcap = d_cap;
+          nodes = reinterpret_cast<const float4*>((uintptr_t)(((uint64_t)d_nhi << 32) | d_nlo));
+          sid = d_sid;
+          fl = kfHelper | kfSplit | kfLevel | kfWt | (d_fl & kfMirror);
+          lbest = d_cap;
+          sp = base = tsp = mark = 0;
+          cur = tn > (!ANY && at < d_mark ? d_cull0 : cullb) ? kNone : ref;
+          mode = (cur != kNone && (cur & kLeafBit)) ? kLeaf : kNode;
+          atomicAdd(&helpers[wbase + own], 1u);
+        }
+      }
+    }
+    if (!__any(mode != kIdle)) break;
+
+    if (exhausted)
+      run(std::true_type{}, kHelpSteps);
+    else
+      run(std::false_type{}, p.steps);
   }
 }
 

@@ -228,7 +228,7 @@ std::string build_environment(const vt_environment& env, EnvTable& t) {
 // Per-scene shading data.  vt_set_scene builds and uploads a complete set
 // before it binds anything, so a failure leaves the previous scene's set.
 struct RenderSceneData {
-  DeviceBuffer materials, emitters, instances, env_cdf, env_texels, tri_source, light_tree, lights;
+  DeviceBuffer materials, emitters, instances, env_cdf, env_texels, tri_source, light_tree, light_nodes, lights;
   uint32_t n_dir = 0, n_point = 0, n_spot = 0, n_rect = 0;  // analytic emitters in `lights`
   uint32_t light_tree_nodes = 0;  // 0: uniform light selection
   std::vector<float> light_tree_host;
@@ -238,7 +238,7 @@ struct RenderSceneData {
   float ray_bias = 0, tmin = 0;
   float scene_min[3] = {0, 0, 0}, scene_inv_extent[3] = {1, 1, 1};
   void release_scene() {
-    for (DeviceBuffer* b : {&materials, &emitters, &instances, &env_cdf, &env_texels, &tri_source, &light_tree, &lights})
+    for (DeviceBuffer* b : {&materials, &emitters, &instances, &env_cdf, &env_texels, &tri_source, &light_tree, &light_nodes, &lights})
       b->release();
   }
 };
@@ -536,6 +536,10 @@ vt_status engine_prepare_render(vt_engine* e, const vt::Pack& P, const std::vect
   s = s ? s : engine_upload(e, R.env_texels, et.texels.data(), et.texels.size() * 4);
   s = s ? s : engine_upload(e, R.tri_source, P.tri_source.data(), P.tri_source.size() * 4);
   s = s ? s : engine_upload(e, R.light_tree, tree.data(), tree.size() * 4);
+  s = s ? s : R.light_nodes.ensure(e, std::max<size_t>((size_t)R.light_tree_nodes * 64, 64));
+  if (!s)
+    HIP_CHECK(e, vtr::launch_light_prepare((const float*)R.light_tree.ptr, R.light_tree_nodes,
+                                           (float4*)R.light_nodes.ptr, e->stream));
   if (ana.records.empty()) ana.records.assign(vtr::kLightFloats, 0.0f);
   s = s ? s : engine_upload(e, R.lights, ana.records.data(), ana.records.size() * 4);
   if (!s && (e->fail_inject & kInjectRenderAlloc)) {
@@ -669,7 +673,7 @@ static vt_status frame_setup(vt_engine* e, const vt_frame* fr, FrameLaunch& L) {
   sc.env_h = R.env_h;
   sc.env_rot_c = R.env_rot[0];
   sc.env_rot_s = R.env_rot[1];
-  sc.light_tree = (const float*)R.light_tree.ptr;
+  sc.light_nodes = (const float4*)R.light_nodes.ptr;
   sc.light_tree_nodes = R.light_tree_nodes;
   sc.lights = (const float*)R.lights.ptr;
   sc.n_dir = R.n_dir;

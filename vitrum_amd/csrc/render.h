@@ -31,8 +31,9 @@ struct ShadeScene {
   uint32_t emitter_count;
   uint32_t env_present, env_w, env_h;
   float env_rot_c, env_rot_s;   // the dome's rotation about +Y
-  // Light tree over the light slots (16 floats per node); 0 nodes = uniform.
-  const float* light_tree;
+  // Light tree over the light slots as the descent reads it (4 float4s per
+  // node, launch_light_prepare); 0 nodes = uniform.
+  const float4* light_nodes;
   uint32_t light_tree_nodes;
   // Analytic emitters (kLightFloats each) in light-selection order:
   // directional, point, spot, then rect and disc areas; the mesh-area
@@ -124,6 +125,9 @@ struct PathState {
   float* train_tgt;       // 3 per training sample
 };
 
+// Derives the descent's nodes (4 float4s each) from a packed light tree (16
+// floats per node) on the device; once per scene.
+hipError_t launch_light_prepare(const float* tree, uint32_t nodes, float4* out, hipStream_t st);
 hipError_t launch_camera(const FrameParams& f, const PathState& s, hipStream_t st);
 hipError_t launch_shade(const FrameParams& f, const ShadeScene& sc, const PathState& s,
                         uint32_t vertex, uint32_t capacity, hipStream_t st);

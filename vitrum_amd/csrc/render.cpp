@@ -228,17 +228,20 @@ std::string build_environment(const vt_environment& env, EnvTable& t) {
 // Per-scene shading data.  vt_set_scene builds and uploads a complete set
 // before it binds anything, so a failure leaves the previous scene's set.
 struct RenderSceneData {
-  DeviceBuffer materials, emitters, instances, env_cdf, env_texels, tri_source, light_tree, light_nodes, lights;
+  DeviceBuffer materials, emitters, instances, env_cdf, env_texels, env_row_cos, tri_source, light_tree,
+      light_nodes, lights;
   uint32_t n_dir = 0, n_point = 0, n_spot = 0, n_rect = 0;  // analytic emitters in `lights`
   uint32_t light_tree_nodes = 0;  // 0: uniform light selection
   std::vector<float> light_tree_host;
   uint32_t emitter_count = 0;
+  uint32_t ext_lobes = 0;  // some material has a clearcoat, sheen or anisotropy
   uint32_t env_present = 0, env_w = 0, env_h = 0;
   float env_rot[2] = {1, 0};  // cos, sin of the dome's rotation about +Y
   float ray_bias = 0, tmin = 0;
   float scene_min[3] = {0, 0, 0}, scene_inv_extent[3] = {1, 1, 1};
   void release_scene() {
-    for (DeviceBuffer* b : {&materials, &emitters, &instances, &env_cdf, &env_texels, &tri_source, &light_tree, &light_nodes, &lights})
+    for (DeviceBuffer* b : {&materials, &emitters, &instances, &env_cdf, &env_texels, &env_row_cos, &tri_source,
+                            &light_tree, &light_nodes, &lights})
       b->release();
   }
 };
@@ -390,6 +393,7 @@ vt_status engine_prepare_render(vt_engine* e, const vt::Pack& P, const std::vect
     q[18] = (float)std::sin((double)m.anisotropy_rotation);
     for (int k = 0; k < 3; ++k) q[19 + k] = m.has_specular ? std::max(0.0f, m.specular_color[k]) : 1.0f;
     q[22] = m.has_specular ? c01(m.specular_intensity) : 1.0f;
+    if (q[9] > 0.0f || q[11] > 0.0f || q[16] > 0.0f) R.ext_lobes = 1;
   }
   if (materials.empty()) {
     mats[0] = mats[1] = mats[2] = 0.8f, mats[3] = 1.0f;
@@ -534,6 +538,8 @@ vt_status engine_prepare_render(vt_engine* e, const vt::Pack& P, const std::vect
   if (et.texels.empty()) et.texels.assign(4, 0.0f);
   s = s ? s : engine_upload(e, R.env_cdf, et.cdf.data(), et.cdf.size() * 4);
   s = s ? s : engine_upload(e, R.env_texels, et.texels.data(), et.texels.size() * 4);
+  s = s ? s : R.env_row_cos.ensure(e, ((size_t)et.h + 1) * sizeof(double));
+  if (!s) HIP_CHECK(e, vtr::launch_env_rows(et.h, (double*)R.env_row_cos.ptr, e->stream));
   s = s ? s : engine_upload(e, R.tri_source, P.tri_source.data(), P.tri_source.size() * 4);
   s = s ? s : engine_upload(e, R.light_tree, tree.data(), tree.size() * 4);
   s = s ? s : R.light_nodes.ensure(e, std::max<size_t>((size_t)R.light_tree_nodes * 64, 64));
@@ -667,6 +673,7 @@ static vt_status frame_setup(vt_engine* e, const vt_frame* fr, FrameLaunch& L) {
   sc.instances = (const float*)R.instances.ptr;
   sc.env_cdf = (const float*)R.env_cdf.ptr;
   sc.env_texels = (const float4*)R.env_texels.ptr;
+  sc.env_row_cos = (const double*)R.env_row_cos.ptr;
   sc.emitter_count = R.emitter_count;
   sc.env_present = R.env_present;
   sc.env_w = R.env_w;
@@ -680,6 +687,7 @@ static vt_status frame_setup(vt_engine* e, const vt_frame* fr, FrameLaunch& L) {
   sc.n_point = R.n_point;
   sc.n_spot = R.n_spot;
   sc.n_rect = R.n_rect;
+  sc.ext_lobes = R.ext_lobes;
   vtr::PathState& ps = L.ps;
   ps = vtr::PathState{};
   ps.rng = (uint32_t*)R.rng.ptr;

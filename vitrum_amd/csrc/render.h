@@ -28,6 +28,7 @@ struct ShadeScene {
   const float* instances;       // kInstFloats per packed instance
   const float* env_cdf;         // env_w * env_h + 1
   const float4* env_texels;     // per texel: scaled radiance rgb, pdf per steradian
+  const double* env_row_cos;    // cos(theta) at the env_h + 1 row edges
   uint32_t emitter_count;
   uint32_t env_present, env_w, env_h;
   float env_rot_c, env_rot_s;   // the dome's rotation about +Y
@@ -40,6 +41,7 @@ struct ShadeScene {
   // emitters follow them in the selection index, the environment comes last.
   const float* lights;
   uint32_t n_dir, n_point, n_spot, n_rect;
+  uint32_t ext_lobes;  // some material has a clearcoat, sheen or anisotropy
 };
 
 // Analytic emitter records (16 floats; no_shadow = castShadow false):
@@ -128,6 +130,8 @@ struct PathState {
 // Derives the descent's nodes (4 float4s each) from a packed light tree (16
 // floats per node) on the device; once per scene.
 hipError_t launch_light_prepare(const float* tree, uint32_t nodes, float4* out, hipStream_t st);
+// cos(theta) at the h + 1 row edges of an environment map; once per scene.
+hipError_t launch_env_rows(uint32_t h, double* out, hipStream_t st);
 hipError_t launch_camera(const FrameParams& f, const PathState& s, hipStream_t st);
 hipError_t launch_shade(const FrameParams& f, const ShadeScene& sc, const PathState& s,
                         uint32_t vertex, uint32_t capacity, hipStream_t st);

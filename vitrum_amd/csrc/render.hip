@@ -23,6 +23,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "fast_div.h"
@@ -93,26 +94,29 @@ __device__ __forceinline__ uint32_t pcg_next(uint32_t& s) {
   return (w >> 22) ^ w;
 }
 // Per-path sampler: PCG (dim == kPcgOnly) or pt-webgpu's Owen-scrambled
-// Sobol stream, which continues with PCG after its last dimension.
+// Sobol stream, which continues with PCG after its last dimension.  A kernel
+// built without SOBOL draws from PCG alone.
 constexpr uint32_t kPcgOnly = 0xFFFFFFFFu;
+template <bool SOBOL>
 struct Rng {
   uint32_t s;     // PCG state / Sobol continuation state
   uint32_t dim;   // next Sobol dimension, kPcgOnly for PCG
-  uint32_t seed;  // Sobol stream seed (pixel and sequence key)
-  uint32_t tile;  // Sobol rotation tile
-  uint32_t sample;
+  vts::Stream st; // Sobol stream of the pixel and sequence key
   const uint16_t* dirs;
 };
-__device__ __forceinline__ uint32_t rng_next(Rng& r) {
+template <bool SOBOL>
+__device__ __forceinline__ uint32_t rng_next(Rng<SOBOL>& r) {
+  if (!SOBOL) return pcg_next(r.s);
   if (r.dim >= vts::kDims) {
     if (r.dim != kPcgOnly) ++r.dim;
     return pcg_next(r.s);
   }
-  const uint32_t v = vts::owen_u32(r.dirs, r.sample, r.dim, r.tile, r.seed);
+  const uint32_t v = vts::stream_u32(r.dirs, r.st, r.dim);
   ++r.dim;
   return v;
 }
-__device__ __forceinline__ float rand01(Rng& r) { return (float)(rng_next(r) >> 8) / 16777216.0f; }
+template <bool SOBOL>
+__device__ __forceinline__ float rand01(Rng<SOBOL>& r) { return (float)(rng_next(r) >> 8) / 16777216.0f; }
 // Polar disc coordinates sqrt(u1)·cos(2π·u2), sqrt(u1)·sin(2π·u2), evaluated
 // in binary64 and rounded once to binary32.  A phase rounded to binary32
 // first (2π·u2 near 6 carries up to 2.4e-7 rad) and a binary32 cosine would
@@ -131,7 +135,8 @@ __device__ float represented(float p) {
   const float b = clampf(floorf(p * 16777216.0f + 0.5f), 1.0f, 16777215.0f);
   return b / 16777216.0f;
 }
-__device__ uint32_t rand_bounded(Rng& s, uint32_t bound) {
+template <bool SOBOL>
+__device__ uint32_t rand_bounded(Rng<SOBOL>& s, uint32_t bound) {
   if (bound <= 1u) return 0u;
   const uint32_t threshold = ((0xFFFFFFFFu % bound) + 1u) % bound;
   for (;;) {
@@ -315,9 +320,14 @@ __device__ __forceinline__ float lt_importance(const LtNode& n, F3 p) {
 // sampleLightTree: one 24-bit root draw apportioned down the tree (every leaf
 // keeps one bucket, the spare buckets follow the represented importances).
 // Returns the light slot, or -1; *pdf = leaf buckets / 2^24.
-__device__ int lt_sample(const float4* tree, uint32_t nodes, F3 p, Rng& rng, float* pdf) {
+template <bool SOBOL>
+__device__ __forceinline__ int lt_sample(const float4* tree, uint32_t nodes, F3 p, Rng<SOBOL>& rng, float* pdf) {
   *pdf = 0.0f;
-  LtNode node = lt_load(tree, 0);
+  struct { int left, right; } node;
+  {
+    const float4 d = tree[3];
+    node.left = (int)__float_as_uint(d.y), node.right = (int)__float_as_uint(d.z);
+  }
   uint32_t cur = 0x01000000u, local = 0;
   if (node.left >= 0) local = min(0x00FFFFFFu, rng_next(rng) >> 8);
   for (uint32_t guard = 0; guard < nodes + 1u; ++guard) {
@@ -325,9 +335,21 @@ __device__ int lt_sample(const float4* tree, uint32_t nodes, F3 p, Rng& rng, flo
       *pdf = (float)cur / 16777216.0f;
       return node.right;
     }
-    const LtNode l = lt_load(tree, (uint32_t)node.left), r = lt_load(tree, (uint32_t)node.right);
-    const float li = lt_importance(l, p), ri = lt_importance(r, p);
-    const uint32_t remaining = cur - (l.count + r.count);
+    // one copy of the importance for both children: the registers of two at
+    // once would cost a wave per SIMD
+    const uint32_t kids[2] = {(uint32_t)node.left, (uint32_t)node.right};
+    float imp[2];
+    uint32_t count[2];
+    int next[2][2];
+#pragma unroll 1
+    for (int c = 0; c < 2; ++c) {
+      const LtNode k = lt_load(tree, c ? kids[1] : kids[0]);
+      const float v = lt_importance(k, p);
+      imp[1] = v, count[1] = k.count, next[1][0] = k.left, next[1][1] = k.right;
+      if (c == 0) imp[0] = v, count[0] = k.count, next[0][0] = k.left, next[0][1] = k.right;
+    }
+    const float li = imp[0], ri = imp[1];
+    const uint32_t remaining = cur - (count[0] + count[1]);
     float p_left = 0.5f;
     const float s = fmaxf(li, ri);
     if (s > 0.0f) {
@@ -335,15 +357,12 @@ __device__ int lt_sample(const float4* tree, uint32_t nodes, F3 p, Rng& rng, flo
       p_left = lf / (lf + rf);
     }
     const float rounded = floorf((float)remaining * p_left + 0.5f);
-    const uint32_t left = l.count + min(remaining, (uint32_t)fmaxf(0.0f, rounded));
-    if (local < left) {
-      cur = left;
-      node = l;
-    } else {
-      local -= left;
-      cur -= left;
-      node = r;
-    }
+    const uint32_t left = count[0] + min(remaining, (uint32_t)fmaxf(0.0f, rounded));
+    const bool go_left = local < left;
+    local = go_left ? local : local - left;
+    cur = go_left ? left : cur - left;
+    node.left = go_left ? next[0][0] : next[1][0];
+    node.right = go_left ? next[0][1] : next[1][1];
   }
   return -1;
 }
@@ -752,17 +771,79 @@ __device__ float bsdf_pdf(const Mat& m, F3 n, F3 wo, F3 wi) {
   return (e.base * base + e.cc * cc_pdf(m, n, wo, wi)) + e.sheen * sheen_pdf(m, n, wo, wi);
 }
 
+// The BSDF's value and directional density for one pair of directions, and
+// what of them depends on the view alone, computed once per vertex: Fresnel
+// end points, the specular probability, the view's masking and Kulla-Conty
+// terms.  Both vanish under the same condition (|N.V| or |N.L| <= 1e-5 or
+// below the surface) and share the half vector and the GGX density.  With EXT
+// the extension lobes go through bsdf_eval and bsdf_pdf; a scene without
+// them runs the kernel without.
+struct View {
+  F3 f0, fms;
+  float f90, sp, ndv, alpha, g1, eo, om;
+};
+template <bool EXT>
+__device__ __forceinline__ View view_of(const Mat& m, F3 n, F3 wo) {
+  View v;
+  v.ndv = fmaxf(dot(n, wo), 0.0f);
+  v.f0 = spec_f0(m);
+  v.f90 = spec_f90(m);
+  const F3 F = schlick01(v.ndv, v.f0, v.f90);
+  v.sp = represented(clampf(0.04f + (0.96f - 0.04f) * fmaxf(luminance(F), m.metal), 0.04f, 0.96f));
+  if (!EXT) {
+    v.alpha = fmaxf(m.rough * m.rough, 1e-3f);
+    v.g1 = smith_g1(v.ndv, m.rough);
+    const float eavg = lut_eavg(m.rough);
+    v.om = 1.0f - eavg;
+    v.eo = lut_e(v.ndv, m.rough);
+    const float c[3] = {clampf(v.f0.x, 0, 1), clampf(v.f0.y, 0, 1), clampf(v.f0.z, 0, 1)};
+    float o[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float favg = c[k] + (1.0f - c[k]) * (1.0f / 21.0f);
+      o[k] = favg * favg * eavg / fmaxf(1.0f - favg * v.om, 1e-4f);
+    }
+    v.fms = f3(o[0], o[1], o[2]);
+  }
+  return v;
+}
+template <bool EXT>
+__device__ __forceinline__ F3 bsdf_both(const Mat& m, const View& v, F3 n, F3 wo, F3 wi, float& pdf) {
+  if (EXT) {
+    pdf = bsdf_pdf(m, n, wo, wi);
+    return bsdf_eval(m, n, wo, wi);
+  }
+  pdf = 0.0f;
+  const float ndl = fmaxf(dot(n, wi), 0.0f), ndv = v.ndv;
+  if (ndl <= 1e-5f || ndv <= 1e-5f) return f3(0, 0, 0);
+  const F3 h = safe_normalize(wi + wo);
+  const float vdh = fmaxf(dot(wo, h), 0.0f);
+  const F3 F = schlick01(vdh, v.f0, v.f90);
+  const float kdm = 1.0f - m.metal;
+  const F3 diff = f3((1.0f - F.x) * kdm * m.base.x * kInvPi, (1.0f - F.y) * kdm * m.base.y * kInvPi,
+                     (1.0f - F.z) * kdm * m.base.z * kInvPi);
+  const float d = ggx_d(n, h, v.alpha);
+  const float g = v.g1 * smith_g1(ndl, m.rough);
+  const F3 spec = (d * g) * F * (1.0f / fmaxf(4.0f * ndv * ndl, 1e-6f));
+  F3 ms = f3(0, 0, 0);
+  if (!(v.om < 1e-4f)) {
+    const float ei = lut_e(ndl, m.rough);
+    const float shape = (1.0f - v.eo) * (1.0f - ei) / fmaxf(kPi * v.om, 1e-6f);
+    ms = v.fms * shape;
+  }
+  const float pspec = (d * v.g1) / fmaxf(4.0f * ndv, 1e-6f);
+  pdf = (1.0f - v.sp) * (ndl * kInvPi) + v.sp * pspec;
+  return diff + spec + ms;
+}
+
 // sampleGgxVndfTangent (bsdf.wgsl.ts:1710-1735) and, with ax != ay,
-// sampleGgxVndfAnisTangent (bsdf.wgsl.ts:612-637).
-__device__ F3 vndf_sample(F3 wo, float ax, float ay, Rng& rng) {
+// sampleGgxVndfAnisTangent (bsdf.wgsl.ts:612-637), from a polar disc point.
+__device__ __forceinline__ F3 vndf_sample(F3 wo, float ax, float ay, float a, float b) {
   const F3 vh = safe_normalize(f3(ax * wo.x, ay * wo.y, wo.z));
   const float lensq = vh.x * vh.x + vh.y * vh.y;
   const float inv = lensq > 1e-10f ? 1.0f / __builtin_sqrtf(lensq) : 0.0f;
   const F3 t1 = lensq > 1e-10f ? f3(-vh.y * inv, vh.x * inv, 0.0f) : f3(1, 0, 0);
   const F3 t2 = cross(vh, t1);
-  const float u1 = rand01(rng), u2 = rand01(rng);
-  float a, b;
-  disc_polar(u1, u2, a, b);
   const float s = 0.5f * (1.0f + vh.z);
   b = (1.0f - s) * __builtin_sqrtf(fmaxf(0.0f, 1.0f - a * a)) + s * b;
   const F3 nh = a * t1 + b * t2 + __builtin_sqrtf(fmaxf(0.0f, 1.0f - a * a - b * b)) * vh;
@@ -829,31 +910,39 @@ __device__ float4 env_lookup(const ShadeScene& sc, F3 wd) {
 // A direction inside environment texel (x, y), uniform in phi and cos(theta)
 // (environmentPacking.ts texel layout), evaluated in binary64 and rounded once
 // per component, as the binary64 restatement rounds it.
-__device__ F3 env_cell_dir(uint32_t x, uint32_t y, uint32_t w, uint32_t h, float xa, float xb) {
-  const double kTwoPi = 6.283185307179586, kPiD = 3.141592653589793;
+__device__ F3 env_cell_dir(const double* row_cos, uint32_t x, uint32_t y, uint32_t w, float xa, float xb) {
+  const double kTwoPi = 6.283185307179586;
   const double phi0 = ((double)x / w - 0.5) * kTwoPi, phi1 = ((double)(x + 1u) / w - 0.5) * kTwoPi;
-  const double th0 = (double)y / h * kPiD, th1 = (double)(y + 1u) / h * kPiD;
   const double phi = phi0 + (phi1 - phi0) * (double)xa;
-  const double c0 = cos(th0), c1 = cos(th1);
+  const double c0 = row_cos[y], c1 = row_cos[y + 1u];
   const double ct = c0 + (c1 - c0) * (double)xb;
   const double st = __builtin_sqrt(fmax(0.0, 1.0 - ct * ct));
   double sp, cp;
   sincos(phi, &sp, &cp);
   return f3((float)(cp * st), (float)ct, (float)(sp * st));
 }
+// cos(theta) at the h + 1 edges of the texel rows, once per scene.
+__global__ void env_rows_kernel(uint32_t h, double* __restrict__ out) {
+  const uint32_t y = blockIdx.x * blockDim.x + threadIdx.x;
+  if (y <= h) out[y] = cos((double)y / h * 3.141592653589793);
+}
 
 // ---- analytic emitters (kernel.wgsl.ts:903-918, 1198-1497) --------------------
 
 // cos and sin of a binary32 angle, evaluated in binary64 and rounded once (the
 // binary64 restatement rounds the same values).
-__device__ __forceinline__ void cos_sin_f(float a, float& c, float& s) {
+__device__ __noinline__ float2 cos_sin_call(float a) {
   double sd, cd;
   sincos((double)a, &sd, &cd);
-  c = (float)cd;
-  s = (float)sd;
+  return make_float2((float)cd, (float)sd);
+}
+__device__ __forceinline__ void cos_sin_f(float a, float& c, float& s) {
+  const float2 r = cos_sin_call(a);
+  c = r.x;
+  s = r.y;
 }
 // x^y evaluated in binary64 and rounded once.
-__device__ __forceinline__ float pow_f(float x, float y) { return (float)pow((double)x, (double)y); }
+__device__ __noinline__ float pow_f(float x, float y) { return (float)pow((double)x, (double)y); }
 __device__ __forceinline__ F3 normalize_f(F3 v) {
   const float l = __builtin_sqrtf(dot(v, v));
   return f3(v.x / l, v.y / l, v.z / l);
@@ -867,10 +956,9 @@ __device__ bool cone_is_delta(float ad) {
 }
 // sampleDirectionalCone (kernel.wgsl.ts:903-918) with ptDirectionalConeSinCos
 // (material.wgsl.ts:224-235): uniform in solid angle inside the cone.
-__device__ F3 sample_directional_cone(F3 axis, float ad, Rng& rng) {
+__device__ __forceinline__ F3 sample_directional_cone(F3 axis, float ad, bool delta, float xi1, float xi2) {
   F3 d = safe_normalize(axis);
-  if (!cone_is_delta(ad)) {
-    const float xi1 = rand01(rng), xi2 = rand01(rng);
+  if (!delta) {
     float cq, sq;
     cos_sin_f(ad * 0.25f, cq, sq);
     const float one_minus_cos_half = (2.0f * sq) * sq;
@@ -1032,18 +1120,16 @@ __device__ __forceinline__ uint32_t train_pixel(const FrameParams& f, uint32_t p
 
 // Sampler of a path (the state word `s` is set by the caller): Sobol for
 // image paths in Sobol mode (pcgInit of common.wgsl.ts:130-150), else PCG.
-__device__ __forceinline__ Rng path_rng(const FrameParams& f, uint32_t px, uint32_t py, bool train) {
-  Rng r;
+template <bool SOBOL>
+__device__ __forceinline__ Rng<SOBOL> path_rng(const FrameParams& f, uint32_t px, uint32_t py, bool train) {
+  Rng<SOBOL> r;
   r.s = 0;
   r.dirs = f.sobol_dirs;
-  r.sample = f.sobol_key & 0xFFFFu;
-  if (f.sobol && !train) {
+  r.dim = kPcgOnly;
+  if (SOBOL && !train) {
     r.dim = 0;
-    r.seed = vts::hash(vts::combine(vts::pixel_seed(px, py), f.sobol_key >> 16));
-    r.tile = (px & 7u) | ((py & 7u) << 3);
-  } else {
-    r.dim = kPcgOnly;
-    r.seed = r.tile = 0;
+    r.st = vts::stream_of(f.sobol_key & 0xFFFFu, (px & 7u) | ((py & 7u) << 3),
+                          vts::hash(vts::combine(vts::pixel_seed(px, py), f.sobol_key >> 16)));
   }
   return r;
 }
@@ -1061,6 +1147,7 @@ __device__ __forceinline__ FrameParams frame_of(const FrameParams& f0) {
   return f;
 }
 
+template <bool SOBOL>
 __global__ void camera_kernel(FrameParams f0, PathState s) {
   const FrameParams f = frame_of(f0);
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1075,8 +1162,8 @@ __global__ void camera_kernel(FrameParams f0, PathState s) {
     s.train_n[p - f.pixels] = 0u;
   }
   const uint32_t px = pix % f.width, py = pix / f.width;
-  Rng rng = path_rng(f, px, py, train);
-  rng.s = train || !f.sobol ? pcg_init(px, py, key) : vts::fallback_init(px, py, f.sobol_key);
+  Rng<SOBOL> rng = path_rng<SOBOL>(f, px, py, train);
+  rng.s = train || !SOBOL ? pcg_init(px, py, key) : vts::fallback_init(px, py, f.sobol_key);
   const float jx = rand01(rng), jy = rand01(rng);
   const float u = ((float)px + jx) / (float)f.width, v = ((float)py + jy) / (float)f.height;
   const float nx = u * 2.0f - 1.0f, ny = 1.0f - v * 2.0f;
@@ -1120,6 +1207,24 @@ __global__ void camera_kernel(FrameParams f0, PathState s) {
 // One vertex of every queued path: MIS connection of the previous BSDF sample,
 // emission, NEE (enqueues a shadow ray), BSDF sample (enqueues the next
 // extension ray) and Russian roulette.
+//
+// Bound by VALU issue and by latency: a vertex is a long chain of dependent
+// loads (queue, hit, material, triangle, light) and divergent branches, so
+// what counts is how many waves a SIMD can hold against it and how often a
+// branch's code is walked.  Each piece of code therefore appears once: every
+// kind of light leaves a direction, a radiance and a weight and one BSDF
+// evaluation follows; every lobe samples through one VNDF; the environment is
+// looked up at one place; rarely reached functions (pow, cos and sin in
+// binary64) are calls.  The kernel is built per sampler and with or without
+// the extension lobes (clearcoat, sheen, anisotropy), so that the usual scene
+// carries neither.  That took it from 276 registers (one wave per SIMD) to
+// 128.  One workgroup shades 256 entries and takes its places in the next
+// queues with one addition each.
+// Measured, with the same images (start, three and four waves per SIMD): a
+// 1080p frame of the box 48.5, 38.5 and 37.6 ms; the 1M-triangle scene, Sobol
+// sampler and sky 9.5, 7.75 and 7.7 ms.
+constexpr int kShadeWaves = 4;
+
 // Material sort (f.shade_sort).  Each workgroup shades its 256 queue entries
 // in the order of a counting sort by a small key -- misses first, then hits
 // grouped by material (ids past 13 share the last group), entries past the
@@ -1130,16 +1235,20 @@ __global__ void camera_kernel(FrameParams f0, PathState s) {
 // diverge, and on the 1080p Cornell frames the sort cost 2-3% of the frame.
 constexpr uint32_t kSortBins = 16;
 
-__global__ __launch_bounds__(256) void shade_kernel(FrameParams f0, ShadeScene sc, PathState s,
+template <bool SOBOL, bool EXT>
+__global__ __launch_bounds__(256, kShadeWaves) void shade_kernel(FrameParams f0, ShadeScene sc, PathState s,
                                                      uint32_t vertex) {
   const FrameParams f = frame_of(f0);
   __shared__ uint32_t s_count[4][kSortBins];
   __shared__ uint16_t s_order[256];
-  const uint32_t n = s.count[0];
-  const uint32_t stride = gridDim.x * blockDim.x;
+  __shared__ uint32_t s_append[2][4], s_base[2];
+  // One workgroup per 256 entries of the queue's capacity; those past its end
+  // leave at once.
+  const uint32_t n = s.count[0], base = blockIdx.x * 256u;
+  if (base >= n) return;
   const uint32_t li = threadIdx.x, wave = li >> 6, lane = li & 63u;
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64u - lane));
-  for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
+  {
     if (f.shade_sort) {
       uint32_t bin = kSortBins - 1u;
       if (base + li < n) {
@@ -1173,13 +1282,13 @@ __global__ __launch_bounds__(256) void shade_kernel(FrameParams f0, ShadeScene s
       const bool miss = inst == kMiss;
       const float4 rb = s.rays[2 * (size_t)i + 1];
       const F3 dir = f3(rb.x, rb.y, rb.z);
-      Rng rng;
+      Rng<SOBOL> rng;
       {
         const bool train = p >= f.pixels;
-        const uint32_t pix = train ? train_pixel(f, p) : p;
-        rng = path_rng(f, pix % f.width, pix / f.width, train);
+        const uint32_t pix = SOBOL && train ? train_pixel(f, p) : p;
+        rng = path_rng<SOBOL>(f, SOBOL ? pix % f.width : 0u, SOBOL ? pix / f.width : 0u, train);
         rng.s = s.rng[p];
-        rng.dim = s.rng_dim[p];
+        if (SOBOL) rng.dim = s.rng_dim[p];
       }
       F3 T = load3(s.throughput + 3 * (size_t)p);
       const F3 Cn = load3(s.conn + 3 * (size_t)p);
@@ -1237,19 +1346,18 @@ __global__ __launch_bounds__(256) void shade_kernel(FrameParams f0, ShadeScene s
           }
         }
         if (best_pdf > 0.0f) L = L + Cn * best_le * power_heuristic(prev_pdf, best_pdf);
-        if (miss && sc.env_present) {
-          const float4 et = env_lookup(sc, dir);
-          L = L + Cn * f3(et.x, et.y, et.z) * power_heuristic(prev_pdf, et.w);
-        }
       }
       const bool alive = (flags & 1u) != 0u;
       bool done = !alive || vertex >= f.bounce_limit;
+      if (miss && sc.env_present && (prev_mis || !done)) {
+        // the environment: through the previous sample's MIS weight, or seen
+        // directly by a path without one
+        const float4 et = env_lookup(sc, dir);
+        const F3 le = f3(et.x, et.y, et.z);
+        L = prev_mis ? L + Cn * le * power_heuristic(prev_pdf, et.w) : L + T * le;
+      }
       if (!done) sig = mix64(sig, miss ? 0xFFFFFFFFFFFFull : (((uint64_t)inst << 32) | prim));
       if (!done && miss) {
-        if (!prev_mis && sc.env_present) {
-          const float4 et = env_lookup(sc, dir);
-          L = L + T * f3(et.x, et.y, et.z);
-        }
         done = true;
         if (vertex == 0 && p < f.pixels) {
           *(float4*)(s.aux_nd + 4 * (size_t)p) = make_float4(0.5f, 1.0f, 0.5f, 0.0f);
@@ -1313,6 +1421,7 @@ __global__ __launch_bounds__(256) void shade_kernel(FrameParams f0, ShadeScene s
           }
         }
         if (!query) {
+        const View view = view_of<EXT>(m, nrm, wo);
         // 3. NEE over one light picked by the light tree, or uniformly when
         //    the tree is off or declines (mediumNee.wgsl.ts:14-38;
         //    kernel.wgsl.ts:1496-1690).
@@ -1334,126 +1443,96 @@ __global__ __launch_bounds__(256) void shade_kernel(FrameParams f0, ShadeScene s
             inv_sel = (float)n_light;
           }
           sig = mix64(sig, 0xA000000000ull | picked);
-          // A shadow ray carries the contribution; a light with castShadow
-          // false adds it unoccluded.
-          auto queue_shadow = [&](F3 contrib, F3 origin, F3 wi, float tmax, bool no_shadow) {
-            if (no_shadow) {
-              L = L + contrib;
-              return;
-            }
-            shadow_c = contrib;
-            shadow_a = make_float4(origin.x, origin.y, origin.z, f.tmin);
-            shadow_b = make_float4(wi.x, wi.y, wi.z, tmax);
-            want_shadow = true;
-          };
-          if (picked < n_ana) {
-            const float* q = sc.lights + (size_t)picked * kLightFloats;
-            const F3 neg_n = f3(-nrm.x, -nrm.y, -nrm.z);
-            if (picked < sc.n_dir) {
-              // directional: irradiance along a (cone-sampled) direction
-              const F3 wi = sample_directional_cone(load3(q), q[3], rng);
-              const F3 off = dot(nrm, wi) > 0.0f ? nrm : neg_n;
-              const float ndl = fabsf(dot(nrm, wi));
-              const F3 fr = bsdf_eval(m, nrm, wo, wi);
-              queue_shadow(T * fr * load3(q + 4) * (ndl * inv_sel), hp + off * f.ray_bias, wi, f32_max(),
-                           q[7] > 0.5f);
-            } else if (picked < sc.n_dir + sc.n_point + sc.n_spot) {
-              // point / spot: delta position, authored decay and cutoff
-              const bool spot = picked >= sc.n_dir + sc.n_point;
-              const float cutoff = q[spot ? 12 : 8], decay = q[spot ? 13 : 9];
-              const F3 tl = load3(q) - hp;
-              const float dist = safe_length(tl);
-              if (dist > 0.0f && !(cutoff > 0.0f && dist > cutoff)) {
-                const F3 wi = f3(tl.x / dist, tl.y / dist, tl.z / dist);
-                float soft = 1.0f;
-                bool lit = true;
-                if (spot) {
-                  const F3 axis = safe_normalize(load3(q + 4));
-                  const float cos_outer = q[7], cos_inner = q[11];
-                  const float cone_cos = dot(f3(-wi.x, -wi.y, -wi.z), axis);
-                  lit = cone_cos >= cos_outer;
-                  soft = smoothstep_f(cos_outer, fmaxf(cos_inner, cos_outer + 1e-6f), cone_cos);
-                }
-                if (lit) {
-                  const F3 off = dot(nrm, wi) > 0.0f ? nrm : neg_n;
-                  const float ndl = fabsf(dot(nrm, wi));
-                  const F3 fr = bsdf_eval(m, nrm, wo, wi);
-                  const float att = point_attenuation(dist, cutoff, decay);
-                  const F3 rad = load3(q + (spot ? 8 : 4));
-                  queue_shadow(T * fr * rad * (ndl * soft * att * inv_sel), hp + off * f.ray_bias, wi,
-                               fmaxf(dist - f.ray_bias * 2.0f, f.tmin), q[3] > 0.5f);
-                }
+          // Every kind of light gives a direction, a radiance and a weight;
+          // the BSDF is evaluated once, after them.  Area lights and the
+          // environment weigh their density `lpdf` against the BSDF's; delta
+          // lights scale by `atten`.
+          F3 wi = f3(0, 1, 0), rad = f3(0, 0, 0);
+          float tmax = f32_max(), lpdf = 0.0f, lden = 1.0f, atten = 1.0f;
+          bool lit = false, mis = false, no_shadow = false;
+          const uint32_t n_delta = sc.n_dir + sc.n_point + sc.n_spot;
+          const bool env_pick = picked >= n_ana + sc.emitter_count;
+          const bool area_pick = picked >= n_delta && !env_pick;
+          const float* q = picked < n_ana ? sc.lights + (size_t)picked * kLightFloats
+                                          : sc.emitters + (size_t)(env_pick ? 0u : picked - n_ana) * kEmitFloats;
+          float xi = 0.0f, xi1 = 0.0f, xi2 = 0.0f;
+          const bool cone = picked < sc.n_dir && !cone_is_delta(q[3]);
+          if (env_pick) xi = rand01(rng);
+          if (env_pick || area_pick || cone) {
+            xi1 = rand01(rng);
+            xi2 = rand01(rng);
+          }
+          if (picked < sc.n_dir) {
+            // directional: irradiance along a (cone-sampled) direction
+            wi = sample_directional_cone(load3(q), q[3], !cone, xi1, xi2);
+            rad = load3(q + 4);
+            no_shadow = q[7] > 0.5f;
+            lit = true;
+          } else if (picked < n_delta) {
+            // point / spot: delta position, authored decay and cutoff
+            const bool spot = picked >= sc.n_dir + sc.n_point;
+            const float cutoff = q[spot ? 12 : 8], decay = q[spot ? 13 : 9];
+            const F3 tl = load3(q) - hp;
+            const float dist = safe_length(tl);
+            if (dist > 0.0f && !(cutoff > 0.0f && dist > cutoff)) {
+              wi = f3(tl.x / dist, tl.y / dist, tl.z / dist);
+              lit = true;
+              if (spot) {
+                const F3 axis = safe_normalize(load3(q + 4));
+                const float cos_outer = q[7], cos_inner = q[11];
+                const float cone_cos = dot(f3(-wi.x, -wi.y, -wi.z), axis);
+                lit = cone_cos >= cos_outer;
+                atten = smoothstep_f(cos_outer, fmaxf(cos_inner, cos_outer + 1e-6f), cone_cos);
               }
+              lden = point_attenuation(dist, cutoff, decay);  // a second factor of delta lights
+              rad = load3(q + (spot ? 8 : 4));
+              tmax = fmaxf(dist - f.ray_bias * 2.0f, f.tmin);
+              no_shadow = q[3] > 0.5f;
+            }
+          } else if (area_pick) {
+            // rect, disc or mesh triangle: a point on the emitter, area measure
+            // to solid angle, MIS against the BSDF
+            const bool mesh = picked >= n_ana;
+            F3 lp, eu, ev;
+            float coef = 0.5f;
+            if (mesh) {
+              const F3 a = load3(q), b = load3(q + 3), c = load3(q + 6);
+              const float su = __builtin_sqrtf(xi1), uu = 1.0f - su, vv = xi2 * su, ww = (1.0f - uu) - vv;
+              lp = a * uu + b * vv + c * ww;
+              eu = b - a;
+              ev = c - a;
+              rad = load3(q + 9);
             } else {
-              // rect / disc area: a point on the emitter, area measure to
-              // solid angle, MIS against the BSDF
-              const F3 c = load3(q), u = load3(q + 4), v = load3(q + 8);
+              const F3 c = load3(q);
+              eu = load3(q + 4), ev = load3(q + 8);
               const bool disc = fabsf(q[15] - 1.0f) < 0.5f;
-              F3 ln;
-              float area;
-              const bool ok = area_measure(u, v, ln, area, disc ? kPi : 4.0f);
-              const float xi1 = rand01(rng), xi2 = rand01(rng);
-              F3 lp;
+              coef = disc ? kPi : 4.0f;
               if (disc) {
                 float dx, dy;
                 concentric_disc(xi1 * 2.0f - 1.0f, xi2 * 2.0f - 1.0f, dx, dy);
-                lp = (c + u * dx) + v * dy;
+                lp = (c + eu * dx) + ev * dy;
               } else {
-                lp = (c + u * (xi1 * 2.0f - 1.0f)) + v * (xi2 * 2.0f - 1.0f);
+                lp = (c + eu * (xi1 * 2.0f - 1.0f)) + ev * (xi2 * 2.0f - 1.0f);
               }
-              const F3 tl = lp - hp;
-              const float dist = safe_length(tl);
-              const F3 wi = safe_normalize(tl);
-              const float ndl = fabsf(dot(nrm, wi));
-              if (dist > 0.0f && ndl > 0.0f && ok) {
-                const float cl = fmaxf(dot(ln, f3(-wi.x, -wi.y, -wi.z)), 0.0f);
-                if (cl > 0.0f) {
-                  const float lpdf = area_to_solid_angle(dist, cl, area, edge_scale(u, v));
-                  if (lpdf > 0.0f) {
-                    const F3 fr = bsdf_eval(m, nrm, wo, wi);
-                    const float bpdf = bsdf_pdf(m, nrm, wo, wi);
-                    const float w = power_heuristic(lpdf, bpdf);
-                    const F3 off = dot(nrm, wi) > 0.0f ? nrm : neg_n;
-                    queue_shadow(T * fr * load3(q + 12) * (ndl * w / lpdf * inv_sel), hp + off * f.ray_bias, wi,
-                                 fmaxf(dist - f.ray_bias * 2.0f, f.tmin), q[3] > 0.5f);
-                  }
-                }
-              }
+              rad = load3(q + 12);
+              no_shadow = q[3] > 0.5f;
             }
-          } else if (picked - n_ana < sc.emitter_count) {
-            const float* e = sc.emitters + (size_t)(picked - n_ana) * kEmitFloats;
-            const F3 a = load3(e), b = load3(e + 3), c = load3(e + 6);
-            const float r1 = rand01(rng), r2 = rand01(rng);
-            const float su = __builtin_sqrtf(r1), uu = 1.0f - su, vv = r2 * su, ww = (1.0f - uu) - vv;
-            const F3 lp = a * uu + b * vv + c * ww;
             const F3 tl = lp - hp;
             const float dist = safe_length(tl);
             F3 ln;
             float area;
-            const bool ok = area_measure(b - a, c - a, ln, area);
-            const F3 wi = safe_normalize(tl);
-            const float ndl = fabsf(dot(nrm, wi));
-            if (dist > 0.0f && ndl > 0.0f && ok) {
-              const F3 fr = bsdf_eval(m, nrm, wo, wi);
+            const bool ok = area_measure(eu, ev, ln, area, coef);
+            wi = safe_normalize(tl);
+            if (dist > 0.0f && ok) {
               float cl = dot(ln, f3(-wi.x, -wi.y, -wi.z));
-              cl = e[12] > 0.5f ? fabsf(cl) : fmaxf(cl, 0.0f);
-              if (cl > 0.0f) {
-                const float lpdf = area_to_solid_angle(dist, cl, area, edge_scale(b - a, c - a));
-                if (lpdf > 0.0f) {
-                  const float bpdf = bsdf_pdf(m, nrm, wo, wi);
-                  const float w = power_heuristic(lpdf, bpdf);
-                  const F3 off = dot(nrm, wi) > 0.0f ? nrm : f3(-nrm.x, -nrm.y, -nrm.z);
-                  const F3 so = hp + off * f.ray_bias;
-                  const float tmax = fmaxf(dist - f.ray_bias * 2.0f, f.tmin);
-                  shadow_c = T * fr * load3(e + 9) * (ndl * w / lpdf * inv_sel);
-                  shadow_a = make_float4(so.x, so.y, so.z, f.tmin);
-                  shadow_b = make_float4(wi.x, wi.y, wi.z, tmax);
-                  want_shadow = true;
-                }
-              }
+              cl = mesh && q[12] > 0.5f ? fabsf(cl) : fmaxf(cl, 0.0f);
+              if (cl > 0.0f) lpdf = area_to_solid_angle(dist, cl, area, edge_scale(eu, ev));
+              lit = lpdf > 0.0f;
             }
+            lden = lpdf;
+            tmax = fmaxf(dist - f.ray_bias * 2.0f, f.tmin);
+            mis = true;
           } else {
-            const float xi = rand01(rng);
             const uint32_t count = sc.env_w * sc.env_h;
             uint32_t lo = 0, hi = count;
             while (lo + 1u < hi) {
@@ -1461,86 +1540,89 @@ __global__ __launch_bounds__(256) void shade_kernel(FrameParams f0, ShadeScene s
               if (sc.env_cdf[mid] <= xi) lo = mid; else hi = mid;
             }
             const uint32_t idx = min(lo, count - 1u);
-            const float xa = rand01(rng), xb = rand01(rng);
             const uint32_t ex = idx % sc.env_w, ey = idx / sc.env_w;
-            const F3 wi = safe_normalize(env_to_world(sc, env_cell_dir(ex, ey, sc.env_w, sc.env_h, xa, xb)));
+            wi = safe_normalize(env_to_world(sc, env_cell_dir(sc.env_row_cos, ex, ey, sc.env_w, xi1, xi2)));
             const float4 et = sc.env_texels[idx];
-            const float epdf = et.w;
-            const F3 env = f3(et.x, et.y, et.z);
-            const float ndl = fabsf(dot(nrm, wi));
-            if (ndl > 0.0f) {
+            lpdf = et.w;
+            lden = fmaxf(lpdf, 1e-8f);
+            rad = f3(et.x, et.y, et.z);
+            mis = true;
+            lit = true;
+          }
+          const float ndl = fabsf(dot(nrm, wi));
+          if (lit && (!mis || ndl > 0.0f)) {
+            float bpdf;
+            const F3 fr = bsdf_both<EXT>(m, view, nrm, wo, wi, bpdf);
+            float weight;
+            if (mis)
+              weight = ndl * power_heuristic(lpdf, bpdf) / lden * inv_sel;
+            else
+              weight = ndl * atten * lden * inv_sel;
+            const F3 contrib = T * fr * rad * weight;
+            if (no_shadow) {
+              // a light with castShadow false adds its contribution unoccluded
+              L = L + contrib;
+            } else {
               const F3 off = dot(nrm, wi) > 0.0f ? nrm : f3(-nrm.x, -nrm.y, -nrm.z);
               const F3 so = hp + off * f.ray_bias;
-              const F3 fr = bsdf_eval(m, nrm, wo, wi);
-              const float bpdf = bsdf_pdf(m, nrm, wo, wi);
-              const float w = power_heuristic(epdf, bpdf);
-              shadow_c = T * fr * env * (ndl * w / fmaxf(epdf, 1e-8f) * inv_sel);
+              shadow_c = contrib;
               shadow_a = make_float4(so.x, so.y, so.z, f.tmin);
-              shadow_b = make_float4(wi.x, wi.y, wi.z, f32_max());
+              shadow_b = make_float4(wi.x, wi.y, wi.z, tmax);
               want_shadow = true;
             }
           }
         }
         // 4. BSDF sample, opaque branch (bsdf.wgsl.ts:2920-2997) and the finite
         //    finalizer (bsdf.wgsl.ts:1863-1926).
-        const float ndv = fmaxf(dot(nrm, wo), 0.0f);
-        const float sp = spec_prob(m, ndv);
-        const ExtProbs ep = ext_probs(m);
-        F3 tb, bb;
-        if (m.aniso > 0.0f)
-          aniso_frame(m, nrm, tb, bb);
-        else
-          build_onb(nrm, tb, bb);
-        const F3 inc = f3(-wo.x, -wo.y, -wo.z);
-        F3 wi;
-        uint32_t lobe;  // 0 diffuse, 1 specular, 2 clearcoat, 3 sheen
-        if (rand01(rng) < ep.base) {
+        const float sp = view.sp;
+        const ExtProbs ep = EXT ? ext_probs(m) : ExtProbs{1.0f, 0.0f, 0.0f, 0.0f};
+        // The lobe (0 diffuse, 1 specular, 2 clearcoat, 3 sheen), then two
+        // draws that every lobe takes as a point on the disc.
+        uint32_t lobe;
+        if (rand01(rng) < ep.base)
           lobe = rand01(rng) < sp ? 1u : 0u;
-          if (lobe == 1u) {
-            // glossyReflectionSample / its anisotropic form (bsdf.wgsl.ts:640-691, 1752-1778)
-            const float alpha = fmaxf(m.rough * m.rough, 1e-3f);
-            float ax = alpha, ay = alpha;
-            if (m.aniso > 0.0f) aniso_axes(alpha, m.aniso, ax, ay);
-            const F3 wl = f3(dot(wo, tb), dot(wo, bb), dot(wo, nrm));
-            const F3 hl = vndf_sample(wl, ax, ay, rng);
-            const F3 hw = safe_normalize(hl.x * tb + hl.y * bb + hl.z * nrm);
-            wi = safe_normalize(inc - hw * (2.0f * dot(hw, inc)));
-          } else {
-            // cosineHemisphereSample (bsdf.wgsl.ts:1648-1664), its own frame
-            F3 tc, bc;
-            build_onb(nrm, tc, bc);
-            const float u1 = rand01(rng), u2 = rand01(rng);
-            float a, b;
-            disc_polar(u1, u2, a, b);
-            const float ct = __builtin_sqrtf(fmaxf(0.0f, 1.0f - u1));
-            wi = safe_normalize(a * tc + b * bc + ct * nrm);
-          }
-        } else if (rand01(rng) < ep.cc_given_ext) {
-          // the clearcoat lobe: an isotropic VNDF sample at the coat roughness
-          lobe = 2u;
-          F3 tc, bc;
-          build_onb(nrm, tc, bc);
-          const float alpha = fmaxf(m.cc_rough * m.cc_rough, 1e-3f);
-          const F3 wl = f3(dot(wo, tc), dot(wo, bc), dot(wo, nrm));
-          const F3 hl = vndf_sample(wl, alpha, alpha, rng);
-          const F3 hw = safe_normalize(hl.x * tc + hl.y * bc + hl.z * nrm);
-          wi = safe_normalize(inc - hw * (2.0f * dot(hw, inc)));
+        else
+          lobe = rand01(rng) < ep.cc_given_ext ? 2u : 3u;
+        const float u1 = rand01(rng), u2 = rand01(rng);
+        float da, db;
+        disc_polar(EXT && lobe == 3u ? 1.0f : u1, u2, da, db);
+        F3 tf, bf;
+        if (EXT && m.aniso > 0.0f && (lobe & 1u))
+          aniso_frame(m, nrm, tf, bf);
+        else
+          build_onb(nrm, tf, bf);
+        F3 wi;
+        if (lobe == 0u) {
+          // cosineHemisphereSample (bsdf.wgsl.ts:1648-1664), its own frame
+          const float ct = __builtin_sqrtf(fmaxf(0.0f, 1.0f - u1));
+          wi = safe_normalize(da * tf + db * bf + ct * nrm);
         } else {
-          // charlieSheenSample (bsdf.wgsl.ts:1665-1700): sin(theta_h) = u1^(1/(1/alpha + 2))
-          lobe = 3u;
-          const float u1 = rand01(rng), u2 = rand01(rng);
-          const float alpha = fmaxf(m.sheen_rough * m.sheen_rough, 1e-3f);
-          const float inv = 1.0f / fmaxf(alpha, 1e-4f);
-          const float sin_h = (float)pow((double)u1, 1.0 / (double)(inv + 2.0f));
-          const float cos_h = __builtin_sqrtf(fmaxf(0.0f, 1.0f - sin_h * sin_h));
-          float c, s;
-          disc_polar(1.0f, u2, c, s);
-          const F3 hw = safe_normalize((sin_h * c) * tb + (sin_h * s) * bb + cos_h * nrm);
+          const F3 inc = f3(-wo.x, -wo.y, -wo.z);
+          F3 hw;
+          if (!EXT || lobe < 3u) {
+            // glossyReflectionSample / its anisotropic form (bsdf.wgsl.ts:640-691,
+            // 1752-1778); the clearcoat is an isotropic VNDF sample at its own
+            // roughness
+            const float rough = lobe == 2u ? m.cc_rough : m.rough;
+            const float alpha = fmaxf(rough * rough, 1e-3f);
+            float ax = alpha, ay = alpha;
+            if (EXT && lobe == 1u && m.aniso > 0.0f) aniso_axes(alpha, m.aniso, ax, ay);
+            const F3 wl = f3(dot(wo, tf), dot(wo, bf), dot(wo, nrm));
+            const F3 hl = vndf_sample(wl, ax, ay, da, db);
+            hw = safe_normalize(hl.x * tf + hl.y * bf + hl.z * nrm);
+          } else {
+            // charlieSheenSample (bsdf.wgsl.ts:1665-1700): sin(theta_h) = u1^(1/(1/alpha + 2))
+            const float alpha = fmaxf(m.sheen_rough * m.sheen_rough, 1e-3f);
+            const float inv = 1.0f / fmaxf(alpha, 1e-4f);
+            const float sin_h = (float)pow((double)u1, 1.0 / (double)(inv + 2.0f));
+            const float cos_h = __builtin_sqrtf(fmaxf(0.0f, 1.0f - sin_h * sin_h));
+            hw = safe_normalize((sin_h * da) * tf + (sin_h * db) * bf + cos_h * nrm);
+          }
           wi = safe_normalize(inc - hw * (2.0f * dot(hw, inc)));
         }
         sig = mix64(sig, 0xB0ull + lobe);
-        const float mpdf = bsdf_pdf(m, nrm, wo, wi);
-        const F3 fr = bsdf_eval(m, nrm, wo, wi);
+        float mpdf;
+        const F3 fr = bsdf_both<EXT>(m, view, nrm, wo, wi, mpdf);
         const float cosine = fabsf(dot(nrm, wi));
         const bool allows = mpdf > 0.0f && cosine > 1e-8f;
         const F3 C2 = allows ? T * (fr * (cosine / mpdf)) : f3(0, 0, 0);
@@ -1570,21 +1652,30 @@ __global__ __launch_bounds__(256) void shade_kernel(FrameParams f0, ShadeScene s
         }  // !query
       }
       s.rng[p] = rng.s;
-      s.rng_dim[p] = rng.dim;
+      if (SOBOL) s.rng_dim[p] = rng.dim;
       store3(s.throughput + 3 * (size_t)p, T);
       store3(s.radiance + 3 * (size_t)p, L);
       s.flags[p] = flags;
       s.signature[p] = sig;
     }
-    // Wave-aggregated queue appends (all lanes of the wave reach these).
-    const uint32_t si = wave_append(s.count + 2, want_shadow);
+    // Queue appends: one atomic per workgroup and queue (every thread of the
+    // workgroup reaches these), ranks from wave ballots.
+    const uint64_t m_s = __ballot(want_shadow), m_e = __ballot(want_ext);
+    if (lane == 0) s_append[0][wave] = (uint32_t)__popcll(m_s), s_append[1][wave] = (uint32_t)__popcll(m_e);
+    __syncthreads();
+    if (li < 2u) {
+      const uint32_t* c = s_append[li];
+      s_base[li] = atomicAdd(s.count + 2u - li, c[0] + c[1] + c[2] + c[3]);
+    }
+    __syncthreads();
+    uint32_t si = s_base[0] + (uint32_t)__popcll(m_s & below), ei = s_base[1] + (uint32_t)__popcll(m_e & below);
+    for (uint32_t w = 0; w < wave; ++w) si += s_append[0][w], ei += s_append[1][w];
     if (want_shadow) {
       s.shadow_path[si] = p;
       s.shadow_rays[2 * (size_t)si] = shadow_a;
       s.shadow_rays[2 * (size_t)si + 1] = shadow_b;
       store3(s.shadow_contrib + 3 * (size_t)si, shadow_c);
     }
-    const uint32_t ei = wave_append(s.count + 1, want_ext);
     if (want_ext) {
       s.next_queue[ei] = p;
       s.next_rays[2 * (size_t)ei] = ext_a;
@@ -1811,16 +1902,31 @@ hipError_t launch_light_prepare(const float* tree, uint32_t nodes, float4* out, 
   return hipGetLastError();
 }
 
+hipError_t launch_env_rows(uint32_t h, double* out, hipStream_t st) {
+  hipLaunchKernelGGL(env_rows_kernel, dim3(h / 64 + 1), dim3(64), 0, st, h, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_camera(const FrameParams& f, const PathState& s, hipStream_t st) {
   const uint32_t n = f.pixels + (f.nrc ? f.train_paths : 0u);
-  hipLaunchKernelGGL(camera_kernel, dim3((n + 255) / 256), dim3(256), 0, st, f, s);
+  if (f.sobol)
+    hipLaunchKernelGGL(camera_kernel<true>, dim3((n + 255) / 256), dim3(256), 0, st, f, s);
+  else
+    hipLaunchKernelGGL(camera_kernel<false>, dim3((n + 255) / 256), dim3(256), 0, st, f, s);
   return hipGetLastError();
 }
 
 hipError_t launch_shade(const FrameParams& f, const ShadeScene& sc, const PathState& s,
                         uint32_t vertex, uint32_t capacity, hipStream_t st) {
-  const uint32_t blocks = (capacity + 255) / 256;
-  hipLaunchKernelGGL(shade_kernel, dim3(blocks < 8192 ? blocks : 8192), dim3(256), 0, st, f, sc, s, vertex);
+  const dim3 grid((capacity + 255u) / 256u);
+  if (f.sobol && sc.ext_lobes)
+    hipLaunchKernelGGL((shade_kernel<true, true>), grid, dim3(256), 0, st, f, sc, s, vertex);
+  else if (f.sobol)
+    hipLaunchKernelGGL((shade_kernel<true, false>), grid, dim3(256), 0, st, f, sc, s, vertex);
+  else if (sc.ext_lobes)
+    hipLaunchKernelGGL((shade_kernel<false, true>), grid, dim3(256), 0, st, f, sc, s, vertex);
+  else
+    hipLaunchKernelGGL((shade_kernel<false, false>), grid, dim3(256), 0, st, f, sc, s, vertex);
   return hipGetLastError();
 }
 

@@ -952,22 +952,16 @@ __device__ __forceinline__ bool pair_test(V3 o, V3 dir, const WtRay& w, V3 a, V3
   const float es = fmaxf(fmaxf(fmaxf(fabs_(e1r.x), fabs_(e1r.y)), fmaxf(fabs_(e1r.z), fabs_(e2r.x))),
                          fmaxf(fabs_(e2r.y), fabs_(e2r.z)));
   int side;
-  const float ye = recip_of(es);
-  const V3 s1 = div_by(e1r, es, ye), s2 = div_by(e2r, es, ye);
-  const V3 nr = v3(s1.y * s2.z - s1.z * s2.y, s1.z * s2.x - s1.x * s2.z, s1.x * s2.y - s1.y * s2.x);
-  const float ns = fmaxf(fabs_(nr.x), fmaxf(fabs_(nr.y), fabs_(nr.z)));
-  const bool side_fast = div_den(es) && div_den(ns) && div_den(w.ds) &&
-                         min(min(div_key(e1r), div_key(e2r)), min(div_key(nr), div_key(dir))) >= kDivNum;
-  if (__builtin_expect(side_fast, 1)) {
-    const V3 nd = div_by(nr, ns, recip_of(ns));
-    const float nl = __builtin_sqrtf((nd.x * nd.x + nd.y * nd.y) + nd.z * nd.z);  // in [1, sqrt 3]
-    const V3 n = div_by(nd, nl, recip_of(nl));
-    const V3 d = div_by(dir, w.ds, recip_of(w.ds));
-    const float sd = -((d.x * n.x + d.y * n.y) + d.z * n.z);
-    side = sd == 0.0f ? 0 : (sd > 0.0f ? 1 : -1);
-  } else {
+  // Only the sign of the authored normal along the ray counts.  The reference
+  // normalises both; its rounding and that of this product together stay below
+  // 2^-17 es^2 ds (90 half-ulps of terms at most that large), so a larger
+  // product has the sign already.  Slivers and grazing rays take the long way.
+  const V3 nr = v3(e1r.y * e2r.z - e1r.z * e2r.y, e1r.z * e2r.x - e1r.x * e2r.z, e1r.x * e2r.y - e1r.y * e2r.x);
+  const float along = (dir.x * nr.x + dir.y * nr.y) + dir.z * nr.z;
+  if (__builtin_expect(div_den(es) && div_den(w.ds) && fabs_(along) > ((es * es) * w.ds) * 0x1p-17f, 1))
+    side = along > 0.0f ? -1 : 1;
+  else
     side = wt_side_inl(dir, w.ds, a, b, c);
-  }
   if (side == 0) return false;
   h.front = side > 0;
   h.t = t;
@@ -977,6 +971,15 @@ __device__ __forceinline__ bool pair_test(V3 o, V3 dir, const WtRay& w, V3 a, V3
                          a.z + (h.u * (b.z - a.z) + h.v * (c.z - a.z)))
                     : point;
   return true;
+}
+
+// A 16-byte load through a pointer to global memory.  Of a pointer that comes
+// out of memory the compiler does not know that, and a flat load also waits
+// for LDS.
+typedef float f4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float4 load4(const float4* p) {
+  const f4 v = *(const __attribute__((address_space(1))) f4*)p;
+  return make_float4(v.x, v.y, v.z, v.w);
 }
 
 // ---------------------------------------------------------------------------
@@ -1038,7 +1041,6 @@ constexpr uint32_t kfRefOrder = 4u;    // walking the TLAS in the reference's or
 constexpr uint32_t kfRecheck = 8u;     // two instances' hits came within the margin
 constexpr uint32_t kfLevel = 16u;      // inside an instance
 constexpr uint32_t kfMirror = 32u;     // ... whose local-to-world map reverses orientation
-constexpr uint32_t kfWt = 64u;         // the watertight set-up of the local ray is done
 constexpr uint32_t kfLHit = 128u;      // local hit, and its two bits
 constexpr uint32_t kfLFront = 256u;
 constexpr uint32_t kfLSingle = 512u;
@@ -1046,7 +1048,7 @@ constexpr uint32_t kfSplit = 1024u;    // in a group: an owner with helpers, or 
 constexpr uint32_t kfHelper = 2048u;
 constexpr uint32_t kfTie = 4096u;      // the group met a hit whose fate depends on the order
 constexpr uint32_t kfAlone = 8192u;    // no helpers in this instance (walked again because of kfTie)
-constexpr uint32_t kfLocal = kfLevel | kfMirror | kfWt | kfLHit | kfLFront | kfLSingle | kfSplit | kfTie;
+constexpr uint32_t kfLocal = kfLevel | kfMirror | kfLHit | kfLFront | kfLSingle | kfSplit | kfTie;
 constexpr uint32_t kHelpSteps = 4;     // steps between two rounds of taking work
 
 // Orders a wave's LDS accesses of different lanes (they execute in program
@@ -1063,8 +1065,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
   // Stack entries (child ref, entry distance), entry-major, deeper ones in a
   // per-thread global area; per wave: the pair table of a leaf operation
   // (also the donors' lanes), the groups' best distances and helper counts.
-  __shared__ uint32_t st_ref[D * B];
-  __shared__ float st_tn[D * B];
+  __shared__ uint2 stack[D * B];
   __shared__ uint32_t table[B], group_best[B], helpers[B];
   const uint32_t tid = threadIdx.x, lane = __lane_id(), wbase = tid & ~63u;
   const size_t spill_stride = (size_t)gridDim.x * B, gtid = (size_t)blockIdx.x * B + tid;
@@ -1104,7 +1105,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
     return best;
   };
   auto stk_load = [&](uint32_t i) -> uint2 {
-    if (i < D) return make_uint2(st_ref[i * B + tid], f2u(st_tn[i * B + tid]));
+    if (i < D) return stack[i * B + tid];
     const unsigned long long w = spill[(i - D) * spill_stride + gtid];
     return make_uint2((uint32_t)w, (uint32_t)(w >> 32));
   };
@@ -1182,7 +1183,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
     // one Node128: four child boxes tested axis by axis
     static_assert(kWideKids == 4, "the expansion below is written for 4-wide nodes");
     const float4* nd = nodes + (size_t)kWideNodeFloat4s * cur;
-    float4 a = nd[0], b = nd[3];
+    float4 a = load4(nd), b = load4(nd + 3);
     float n0, n1, n2, n3, f0, f1, f2, f3;
     {
       const float p0 = (a.x - o.x) * inv.x, q0 = (b.x - o.x) * inv.x;
@@ -1194,7 +1195,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
       n2 = fminf(p2, q2), f2 = fmaxf(p2, q2);
       n3 = fminf(p3, q3), f3 = fmaxf(p3, q3);
     }
-    a = nd[1], b = nd[4];
+    a = load4(nd + 1), b = load4(nd + 4);
     {
       const float p0 = (a.x - o.y) * inv.y, q0 = (b.x - o.y) * inv.y;
       const float p1 = (a.y - o.y) * inv.y, q1 = (b.y - o.y) * inv.y;
@@ -1205,7 +1206,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
       n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
       n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
     }
-    a = nd[2], b = nd[5];
+    a = load4(nd + 2), b = load4(nd + 5);
     {
       const float p0 = (a.x - o.z) * inv.z, q0 = (b.x - o.z) * inv.z;
       const float p1 = (a.y - o.z) * inv.z, q1 = (b.y - o.z) * inv.z;
@@ -1216,13 +1217,14 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
       n2 = fmaxf(n2, fminf(p2, q2)), f2 = fminf(f2, fmaxf(p2, q2));
       n3 = fmaxf(n3, fminf(p3, q3)), f3 = fminf(f3, fmaxf(p3, q3));
     }
-    const uint4 r = *reinterpret_cast<const uint4*>(nd + 6);
+    const float4 rf = load4(nd + 6);
+    const uint4 r = make_uint4(f2u(rf.x), f2u(rf.y), f2u(rf.z), f2u(rf.w));
     // What the bound culls and the stack keeps: the entry distance, in a
     // group the near plane on the dominant axis.
     float g0 = n0, g1 = n1, g2 = n2, g3 = n3;
     if (GROUP && (fl & kfSplit)) {
       const int kz = (int)min((lw.perm >> 4) & 3u, 2u);
-      const float4 lo_k = nd[kz], hi_k = nd[3 + kz];
+      const float4 lo_k = load4(nd + kz), hi_k = load4(nd + 3 + kz);
       const float ok = sel3(kz, o.x, o.y, o.z), ik = sel3(kz, inv.x, inv.y, inv.z);
       auto near_plane = [&](float mn, float mx) {
         const float p = (mn - ok) * ik, q = (mx - ok) * ik;
@@ -1257,13 +1259,13 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
     if (__builtin_expect(sp + 4u <= D, 1)) {
       // without branches: each entry is written at the top, which moves
       // past it only when its child is kept
-      st_ref[sp * B + tid] = r.w, st_tn[sp * B + tid] = g3;
+      stack[sp * B + tid] = make_uint2(r.w, f2u(g3));
       sp += u3 ? 1u : 0u;
-      st_ref[sp * B + tid] = r.z, st_tn[sp * B + tid] = g2;
+      stack[sp * B + tid] = make_uint2(r.z, f2u(g2));
       sp += u2 ? 1u : 0u;
-      st_ref[sp * B + tid] = r.y, st_tn[sp * B + tid] = g1;
+      stack[sp * B + tid] = make_uint2(r.y, f2u(g1));
       sp += u1 ? 1u : 0u;
-      st_ref[sp * B + tid] = r.x, st_tn[sp * B + tid] = g0;
+      stack[sp * B + tid] = make_uint2(r.x, f2u(g0));
       sp += u0 ? 1u : 0u;
     } else {
       for (uint32_t c = 4; c-- > 0;) {
@@ -1272,7 +1274,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         const uint32_t ref = c == 3 ? r.w : (c == 2 ? r.z : (c == 1 ? r.y : r.x));
         const float tn = c == 3 ? g3 : (c == 2 ? g2 : (c == 1 ? g1 : g0));
         if (sp < D) {
-          st_ref[sp * B + tid] = ref, st_tn[sp * B + tid] = tn;
+          stack[sp * B + tid] = make_uint2(ref, f2u(tn));
         } else if (sp < kWideStackCapacity) {
           spill[(sp - D) * spill_stride + gtid] = (unsigned long long)ref | ((unsigned long long)f2u(tn) << 32);
         } else {
@@ -1430,6 +1432,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
           }
           o = lo;
           inv = safe_inv3(ld);
+          lw = wt_setup(ld);
           lbest = cullb = lcap;
           fl = (fl & ~kfLocal) | kfLevel | (meta.w != 0u ? kfMirror : 0u);
           nodes = S.blas4_nodes;
@@ -1450,10 +1453,6 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
             cnt = (cur >> 27) & 15u;
             cur = kNone;
             mode = kNode;
-            if (!(fl & kfWt)) {
-              lw = wt_setup(ld);
-              fl |= kfWt;
-            }
           }
           uint32_t excl = 0, total = 0;
 #pragma unroll
@@ -1498,7 +1497,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
             float single = 0.0f;
             if (work) {
               const float4* tr = otris + 3 * (size_t)tri;
-              const float4 w0 = tr[0], w1 = tr[1], w2 = tr[2];
+              const float4 w0 = load4(tr), w1 = load4(tr + 1), w2 = load4(tr + 2);
               single = w2.y;
               hit = pair_test(wo, wd, ww, v3(w0.x, w0.y, w0.z), v3(w0.w, w1.x, w1.y), v3(w1.z, w1.w, w2.x), w_low, w_hi,
                               near && (w_fl & (GROUP ? kfLHit | kfSplit : kfLHit)) == kfLHit, h);
@@ -1514,7 +1513,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
               bool e = false;
               if (hit) {
                 const float4* tr = otris + 3 * (size_t)tri;
-                const float4 w0 = tr[0], w1 = tr[1], w2 = tr[2];
+                const float4 w0 = load4(tr), w1 = load4(tr + 1), w2 = load4(tr + 2);
                 float tn;
                 (void)slab(wo, wi, fminf(w0.x, fminf(w0.w, w1.z)), fminf(w0.y, fminf(w1.x, w1.w)),
                            fminf(w0.z, fminf(w1.y, w2.x)), fmaxf(w0.x, fmaxf(w0.w, w1.z)),
@@ -1654,10 +1653,6 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         // The r-th idle lane takes entry r / n_donors of donor r % n_donors.
         const uint32_t n_don = (uint32_t)__popcll(donors), rank_d = (uint32_t)__popcll(donors & lane_below);
         const uint32_t share = donor && n_idle > rank_d ? (n_idle - rank_d - 1u) / n_don + 1u : 0u;
-        if (donor && !(fl & kfWt)) {
-          lw = wt_setup(ld);
-          fl |= kfWt;
-        }
         if (share != 0u && !(fl & kfSplit)) {
           fl |= kfSplit;
           mark = sp;
@@ -1681,9 +1676,6 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         const float d_low = __shfl(tlow, d), d_cull = __shfl(cullb, d), d_cap = __shfl(lcap, d);
         const float d_cull0 = __shfl(cull0, d);
         const uint32_t d_mark = (uint32_t)__shfl((int)mark, d);
-        const uint64_t d_nodes = (uint64_t)(uintptr_t)nodes;
-        const uint32_t d_nlo = (uint32_t)__shfl((int)(uint32_t)d_nodes, d);
-        const uint32_t d_nhi = (uint32_t)__shfl((int)(uint32_t)(d_nodes >> 32), d);
         const uint32_t d_sid = MULTI ? (uint32_t)__shfl((int)sid, d) : 0u;
         WtRay d_lw;
         d_lw.ds = __shfl(lw.ds, d);
@@ -1694,8 +1686,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         if (donor) base += min(avail, share);
         wave_sync();
         if (got) {
-          const uint32_t ref = st_ref[at * B + wbase + (uint32_t)d];
-          const float tn = st_tn[at * B + wbase + (uint32_t)d];
+          const uint2 e = stack[at * B + wbase + (uint32_t)d];
           own = d_own;
           lw = d_lw;
           o = d_o;
@@ -1704,12 +1695,12 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
           tlow = d_low;
           cullb = d_cull;
           lcap = d_cap;
-          nodes = reinterpret_cast<const float4*>((uintptr_t)(((uint64_t)d_nhi << 32) | d_nlo));
           sid = d_sid;
-          fl = kfHelper | kfSplit | kfLevel | kfWt | (d_fl & kfMirror);
+          nodes = scene_of().blas4_nodes;
+          fl = kfHelper | kfSplit | kfLevel | (d_fl & kfMirror);
           lbest = d_cap;
           sp = base = tsp = mark = 0;
-          cur = tn > (!ANY && at < d_mark ? d_cull0 : cullb) ? kNone : ref;
+          cur = u2f(e.y) > (!ANY && at < d_mark ? d_cull0 : cullb) ? kNone : e.x;
           mode = (cur != kNone && (cur & kLeafBit)) ? kLeaf : kNode;
           atomicAdd(&helpers[wbase + own], 1u);
         }

@@ -103,3 +103,19 @@ def test_grazing_hits_do_not_depend_on_the_group(engine):
                                       first[order].view(np.uint8)), (near, seed)
     finally:
         engine.set_trace_tuning(8, 16, 2, 12)
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1, 63, 64, 65, 4097])
+def test_every_ray_is_handed_out_once(engine, extra):
+    """Queues around the ends of one fill of all waves (the order of the rays
+    changes there) and past it, where the queue's end is transposed."""
+    sc = W.cornell_scene(2048)
+    engine.set_scene(sc)
+    one = W.primary_rays(sc["camera"], 64, 64)[0]
+    for base in (8192, 262144):
+        n = base + extra
+        rays = np.resize(one, n)
+        want = np.resize(engine.trace_closest(one), n)
+        assert np.array_equal(engine.trace_closest(rays).view(np.uint8), want.view(np.uint8)), n
+        occ = engine.trace_any(rays)
+        assert np.array_equal(occ, np.resize(engine.trace_any(one), n)), n

@@ -1025,15 +1025,24 @@ __device__ __forceinline__ float4 load4(const float4* p) {
 // it had then, as the lone walk would have culled them.  Where neither case is
 // met, the nearest triangle is tested and kept in any order.
 //
+// Long rays are neighbours (those along a wall, say), and a wave that holds
+// many of them outlasts the launch.  So where one fill covers the queue a
+// wave's rays are taken n_waves apart, and the last kTailRays per wave of a
+// longer queue are handed out transposed, 64 places apart; the rest goes out
+// in order, for its coherence.  With tails of 0, 64, 128 and 512 rays: the
+// 16-scene batch 1.98, 1.74, 1.73 and 1.83 ms, four 1080p frames of the box
+// 35.8, 34.7, 33.6 and 33.8 ms, shadow rays in the box 1.08 (0) and 0.59 ms
+// (128); the 1M-triangle scene, whose nodes fit no cache, 0.950, 0.956, 0.967
+// and 1.095 ms.  The 256 x 256 frame below: 2.73 -> 2.13 ms.
+//
 // Measured against the same walk without these three (trace_kernel over
-// Node128): 1,677,721 rays of the 1M-triangle scene 1.294 -> 1.033 ms;
+// Node128): 1,677,721 rays of the 1M-triangle scene 1.27 -> 0.97 ms;
 // 419,430 rays of the 32,768-triangle box, one launch after another on three
-// streams, 0.356 -> 0.180 ms and alone 0.99 -> 0.45 ms (its longest ray takes
+// streams, 0.356 -> 0.165 ms and alone 0.99 -> 0.37 ms (its longest ray takes
 // 322 steps, most rays under 60); a 256 x 256 path-traced frame of that box
-// (17 launches of at most 65,536 rays) 7.6 -> 2.9 ms.  Of this, the care that
-// makes a group's closest hit independent of its order costs 0.08 ms and
-// 0.025 ms of the first two; in one step loop for both phases instead of two
-// the first is 1.068 ms.
+// (17 launches of at most 65,536 rays) 7.6 -> 2.13 ms.  The care that makes a
+// group's closest hit independent of its order costs 0.08 ms of the first; in
+// one step loop for both phases instead of two it is 0.04 ms slower.
 constexpr uint32_t kIdle = 0, kNode = 1, kLeaf = 2, kEnter = 3, kExit = 4, kDone = 5;  // what a lane does next
 constexpr uint32_t kfHit = 1u;         // the record holds a hit
 constexpr uint32_t kfReject = 2u;      // ... on the back face of a single-sided material
@@ -1050,6 +1059,7 @@ constexpr uint32_t kfTie = 4096u;      // the group met a hit whose fate depends
 constexpr uint32_t kfAlone = 8192u;    // no helpers in this instance (walked again because of kfTie)
 constexpr uint32_t kfLocal = kfLevel | kfMirror | kfLHit | kfLFront | kfLSingle | kfSplit | kfTie;
 constexpr uint32_t kHelpSteps = 4;     // steps between two rounds of taking work
+constexpr uint32_t kTailRays = 128;    // per wave, of a queue's end
 
 // Orders a wave's LDS accesses of different lanes (they execute in program
 // order; this keeps the compiler from moving them).
@@ -1080,6 +1090,12 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
   const uint32_t take_cap = max(1u, min(64u, n_rays / n_waves + (n_rays % n_waves != 0u)));
   const uint32_t wave_id = blockIdx.x * (B / 64u) + tid / 64u;
   const uint32_t static_end = n_waves * take_cap;
+  // The order in which rays are handed out (see above): `far` apart where one
+  // fill covers them all, and the last `tail` of a longer queue transposed.
+  const bool one_fill = static_end >= n_rays;
+  const uint32_t far = take_cap < 64u ? n_waves : 1u;
+  const uint32_t tail = one_fill ? 0u : min(n_waves * kTailRays, n_rays - static_end) & ~63u;
+  const uint32_t tail_begin = n_rays - tail;
 
   uint32_t mode = kIdle, fl = 0, ray_idx = 0, sid = 0;
   // The current level's ray: origin, reciprocal direction, lower bound, cull
@@ -1605,14 +1621,20 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
     if (!exhausted) {
       if (n_idle >= p.refill_min || n_idle == 64u) {
         const uint32_t take = min(n_idle, take_cap);
-        uint32_t first = wave_id * take_cap;
+        uint32_t first = far == 1u ? wave_id * take_cap : wave_id, step = far;
         if (!first_fill) {
           if (lane == 0) first = static_end + atomicAdd(p.counter, take);
           first = (uint32_t)__shfl((int)first, 0);
+          step = 1u;
         }
+        exhausted = first_fill ? one_fill : first + take >= n_rays;
         first_fill = false;
-        exhausted = first + take >= n_rays;
-        const uint32_t rank = (uint32_t)__popcll(idle & lane_below), idx = first + rank;
+        const uint32_t rank = (uint32_t)__popcll(idle & lane_below);
+        uint32_t idx = first + rank * step;
+        if (tail != 0u && idx >= tail_begin && idx < n_rays) {
+          const uint32_t q = idx - tail_begin;
+          idx = tail_begin + (q & 63u) * (tail >> 6) + (q >> 6);
+        }
         if (mode == kIdle && rank < take && idx < n_rays) {
           ray_idx = idx;
           if (MULTI) {

@@ -65,10 +65,15 @@ __host__ __device__ __forceinline__ uint32_t nmap(uint32_t kb, uint32_t g, uint3
 
 // ---- input encoding (nrcEncoding.ts) --------------------------------------
 
-// a / b from the refined reciprocal y of b, corrected once by the remainder;
-// for operands far from the ends of the range.
+// The encoding's binary32 operations are those of its definition, in its order
+// and each rounded once, so that a cached radiance does not depend on how the
+// work is laid out.
+
+// a / b, correctly rounded, from the refined reciprocal y of b: div_by
+// (fast_div.h) without the step for operands at the ends of the range.
 __device__ __forceinline__ float quotient(float a, float b, float y) {
-  const float q = a * y;
+  float q = a * y;
+  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
   return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
 
@@ -104,26 +109,25 @@ __device__ __forceinline__ void grid_corners(uint32_t l, float nx, float ny, flo
 // octEncodeDir (nrcEncoding.ts): octahedral map of a direction to [0,1]^2.
 __device__ __forceinline__ void oct_encode(float dx, float dy, float dz, float& u, float& v) {
   const float sc = fmaxf(fabsf(dx), fmaxf(fabsf(dy), fabsf(dz)));
-  float px, py;
-  if (__builtin_expect(vtd::div_den(sc), 1)) {
-    // one reciprocal of the sum, each quotient corrected by its remainder
-    const float s = (fabsf(dx) + fabsf(dy)) + fabsf(dz), y = vtd::recip_of(s);
-    px = quotient(dx, s, y);
-    py = quotient(dy, s, y);
-  } else {
-    if (!(sc > 0.0f) || !(sc <= 3.402823e38f)) {
-      u = v = 0.5f;
-      return;
-    }
-    const float sx = dx / sc, sy = dy / sc, sz = dz / sc;
-    const float inv = 1.0f / ((fabsf(sx) + fabsf(sy)) + fabsf(sz));
-    px = sx * inv, py = sy * inv;
+  if (!(sc > 0.0f) || !(sc <= 3.402823e38f)) {
+    u = v = 0.5f;
+    return;
   }
-  if (dz < 0.0f) {
-    const float ox = copysignf(1.0f - fabsf(py), px >= 0.0f ? 1.0f : -1.0f);
-    const float oy = copysignf(1.0f - fabsf(px), py >= 0.0f ? 1.0f : -1.0f);
-    px = ox;
-    py = oy;
+  float sx, sy, sz;
+  const uint32_t key = min(min(vtd::div_key(dx), vtd::div_key(dy)), vtd::div_key(dz));
+  if (__builtin_expect(vtd::div_den(sc) && key >= vtd::kDivNum, 1)) {
+    const float y = vtd::recip_of(sc);
+    sx = quotient(dx, sc, y), sy = quotient(dy, sc, y), sz = quotient(dz, sc, y);
+  } else {
+    sx = dx / sc, sy = dy / sc, sz = dz / sc;
+  }
+  const float s = (fabsf(sx) + fabsf(sy)) + fabsf(sz);  // in [1, 3]
+  const float inv = quotient(1.0f, s, vtd::recip_of(s));
+  float px = sx * inv, py = sy * inv;
+  if (sz < 0.0f) {
+    const float ox = 1.0f - fabsf(py), oy = 1.0f - fabsf(px);
+    px = px >= 0.0f ? ox : -ox;
+    py = py >= 0.0f ? oy : -oy;
   }
   u = px * 0.5f + 0.5f;
   v = py * 0.5f + 0.5f;
@@ -132,25 +136,27 @@ __device__ __forceinline__ void oct_encode(float dx, float dy, float dz, float& 
 // Four of the eight one-blob bins of a scalar (oneBlobEncodeScalar: Gaussian
 // kernels at (i + 0.5) / k, sigma 1/k, normalised to unit L1 over the k
 // bins): the lower or the upper four.  Lane groups 0 and 1 hold the halves of
-// u and 2 and 3 those of v, for the same samples, and add up their sums.
+// u and 2 and 3 those of v, for the same samples, and exchange them.
 __device__ __forceinline__ void one_blob4(float x, uint32_t upper, float* out) {
   const float uc = fminf(fmaxf(x, 0.0f), 1.0f);
   const float c0 = upper ? 4.5f : 0.5f;
-  // exp(-d^2 / 2) = 2^(d^2 k) with k = -log2(e) / 2 in two parts: the product's
-  // low part goes into a factor, so the exponent loses nothing
-  constexpr float kHi = -0x1.715476p-1f, kLo = -0x1.4ae0cp-27f;
-  float sum = 0.0f;
+  float lower[4], higher[4];
 #pragma unroll
   for (uint32_t i = 0; i < 4; ++i) {
-    const float d = __builtin_fmaf(uc, (float)kBlobBins, -(c0 + (float)i)), q = d * d;
-    const float hi = q * kHi, lo = __builtin_fmaf(q, kLo, __builtin_fmaf(q, kHi, -hi));
-    const float e = __builtin_amdgcn_exp2f(hi);  // hi > -41
-    out[i] = __builtin_fmaf(e, lo * 0x1.62e430p-1f, e);
-    sum += out[i];
+    const float d = __builtin_fmaf(uc, (float)kBlobBins, -(c0 + (float)i));  // (uc - centre) * k
+    out[i] = expf(-0.5f * (d * d));
+    // rows of 16 lanes 0 <-> 1 and 2 <-> 3
+    const uint32_t w = __float_as_uint(out[i]);
+    const auto rows = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    lower[i] = __uint_as_float(rows[0]), higher[i] = __uint_as_float(rows[1]);
   }
-  // rows of 16 lanes 0 <-> 1 and 2 <-> 3
-  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
-  sum = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);  // above 2
+  float sum = 0.0f;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) sum += lower[i];
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) sum += higher[i];
+  // From 1.25 (x = 0 or 1, where half of the Gaussian is cut off) to 2.51, and
+  // a bin is at least e^-28.2: every quotient is in the normal range.
   const float y = vtd::recip_of(sum);
 #pragma unroll
   for (uint32_t i = 0; i < 4; ++i) out[i] = quotient(out[i], sum, y);
@@ -177,8 +183,8 @@ __device__ __forceinline__ float2 lds_row(const float2* lds, uint32_t at) {
 }
 
 __device__ __forceinline__ void add_row(float2 t, float w, float& f0, float& f1) {
-  f0 = __builtin_fmaf(w, t.x, f0);
-  f1 = __builtin_fmaf(w, t.y, f1);
+  f0 += w * t.x;
+  f1 += w * t.y;
 }
 
 __device__ __forceinline__ void encode_lane(uint32_t g, const float* f, const float* __restrict__ tables,
@@ -273,6 +279,11 @@ __device__ __forceinline__ void encode_tile(const float* __restrict__ feats, con
     encode_lane(g, f, tables, v, lds);
     B[sb][0] = pack8(v[0]);
     B[sb][1] = pack8(v[1]);
+    // packed here: sunk past the branches of the next block's encoding, the
+    // sixteen unpacked values would wait in registers that then spill
+#pragma unroll
+    for (uint32_t kb = 0; kb < 2; ++kb)
+      asm volatile("" : "+v"(B[sb][kb].x), "+v"(B[sb][kb].y), "+v"(B[sb][kb].z), "+v"(B[sb][kb].w));
   }
 }
 
@@ -325,9 +336,11 @@ __device__ __forceinline__ void output_layer(const uint4* __restrict__ frags, ui
 // memory, so the outputs are those of a direct gather.
 //
 // Bound by VALU issue, with the LDS gathers and MFMAs behind it: a tile takes
-// 2,080 vector instructions beside 136 MFMAs (4,550 with the bf16 rounding
-// written out, eight exponentials a lane and flat gathers).  2,073,600
-// samples: 285 -> 180 us.  Blocks of 512 threads (twice the registers, two
+// 2,370 vector instructions beside 136 MFMAs (4,550 with the bf16 rounding
+// written out, eight exponentials a lane and flat gathers; 2,080 and 3% less
+// time with fused grid sums, a quotient corrected once and a shorter
+// exponential, which changed the last bits of what the cache answers).
+// 2,073,600 samples: 286 -> 185 us.  Blocks of 512 threads (twice the registers, two
 // waves per SIMD) take 217 us.
 
 __global__ __launch_bounds__(kInferBlock) void infer_kernel(const float* __restrict__ feats, uint32_t cap,
@@ -798,9 +811,9 @@ hipError_t launch_pack(const float* master, uint4* frags, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Up to here infer_few_kernel is the faster one (11.3, 15.0, 30.8 and 50.8 us
+// Up to here infer_few_kernel is the faster one (12.1, 15.2, 30.5 and 51.4 us
 // for 4,099, 32,768, 131,072 and 262,144 samples with the host's call, against
-// 31.5, 31.6, 32.7 and 35.6 us): its time grows with the samples, the staged
+// 31.2, 31.6, 32.4 and 34.5 us): its time grows with the samples, the staged
 // kernel's hardly before every CU has its sixteen tiles.
 constexpr uint32_t kFewSamples = 131072;
 

@@ -156,7 +156,7 @@ vtk::DeviceScene engine_device_scene(const SceneBuffers& b, const vt::DeviceLayo
   d.blas4_nodes = (const float4*)b.blas4.ptr;
   d.tlas4_nodes = (const float4*)b.tlas4.ptr;
   d.tlas4_root = L.tlas4_root;
-  if (wide) *wide = !L.blas4_nodes.empty() && L.stack4_need <= vtk::kWideStackCapacity;
+  if (wide) *wide = L.tlas_node_count != 0 && !L.blas4_nodes.empty() && L.stack4_need <= vtk::kWideStackCapacity;
   return d;
 }
 

@@ -556,7 +556,12 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
         }
       }
     }
-    if (!__any(active)) break;
+    if (!__any(active)) {
+      // A scene without instances closes its rays in the refill: the wave is
+      // done only when the supply is.
+      if (exhausted) break;
+      continue;
+    }
 
     for (uint32_t step = 0; step < p.steps; ++step) {
       // ---- deferred expensive work, shared by the lanes that need it ----
@@ -1655,7 +1660,6 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
           fl = 0;
           own = lane;
           restart();
-          if (S.tlas_node_count == 0u) finish(false);  // no TLAS: fail closed
         }
       }
     } else if (idle != 0ull && n_idle != 64u) {
@@ -1728,7 +1732,10 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         }
       }
     }
-    if (!__any(mode != kIdle)) break;
+    if (!__any(mode != kIdle)) {
+      if (exhausted) break;
+      continue;
+    }
 
     if (exhausted)
       run(std::true_type{}, kHelpSteps);

@@ -255,9 +255,12 @@ vt_status vt_set_device_build(vt_engine *eng, uint32_t min_triangles);
  * next matching step fail once -- 1: scene packing throws std::bad_alloc
  * (vt_set_scene on `eng`; vt_pack_scene when `eng` is NULL), 2: the
  * shading-data upload of vt_set_scene reports VT_ERR_OUT_OF_MEMORY, 4: its
- * preparation throws std::runtime_error.  Every entry point catches
- * exceptions and returns VT_ERR_OUT_OF_MEMORY (std::bad_alloc) or
- * VT_ERR_BUILD (any other), so none unwinds into the caller. */
+ * preparation throws std::runtime_error, 8 and 16: the next check of the
+ * traversal's error word (vt_trace_closest, vt_trace_any, vt_capture, a
+ * batch's launch) finds a full stack, or a wave without the helpers it waits
+ * for.  Every entry point catches exceptions and returns VT_ERR_OUT_OF_MEMORY
+ * (std::bad_alloc) or VT_ERR_BUILD (any other), so none unwinds into the
+ * caller. */
 vt_status vt_debug_inject_failure(vt_engine *eng, uint32_t flags);
 
 /* ---- frames ---------------------------------------------------------------- */

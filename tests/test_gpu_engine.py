@@ -49,3 +49,26 @@ def test_failed_set_scene_keeps_the_previous_scene(engine):
         assert np.array_equal(_frame(engine, cornell), img0)
     engine.set_scene(spheres)  # the hooks fired once each; a good scene binds
     assert engine.render_info()["emitter_count"] != info0["emitter_count"]
+
+
+@pytest.mark.parametrize("flag, text", [(8, "stack capacity"), (16, "helpers")])
+def test_each_traversal_error_is_reported_as_what_it_is(engine, flag, text):
+    cornell = W.cornell_scene(2048)
+    rays, _ = W.primary_rays(cornell["camera"], 16, 16, scene_radius=cornell["scene_radius"])
+    engine.set_scene(cornell)
+    _frame(engine, cornell)
+    batch = native.Batch(engine)
+    d_r, d_h = engine.alloc(rays.nbytes), engine.alloc(rays.size * W.HIT_DTYPE.itemsize)
+    try:
+        batch.add_scene(cornell)
+        engine.h2d(d_r, rays)
+        for call in (lambda: engine.trace_closest(rays), lambda: engine.trace_any(rays), lambda: _frame(engine, cornell),
+                     lambda: batch.trace_closest_device(d_r, [0, rays.size], d_h)):
+            engine.inject_failure(flag)
+            with pytest.raises(native.VtError, match=text):
+                call()
+            call()  # reported once
+    finally:
+        batch.close()
+        engine.free(d_r)
+        engine.free(d_h)

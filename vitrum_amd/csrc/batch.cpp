@@ -109,7 +109,8 @@ static vt_status check_overflow(vt_batch* b) {
   uint32_t err = 0;
   B_HIP(b, hipMemcpyAsync(&err, b->eng->error_word.ptr, 4, hipMemcpyDeviceToHost, b->eng->stream));
   B_HIP(b, hipStreamSynchronize(b->eng->stream));
-  if (err) return berr(b, VT_ERR_HIP, "traversal stack capacity exceeded");
+  err = engine_trace_error(b->eng, err);
+  if (err) return berr(b, VT_ERR_HIP, vtk::trace_error_text(err));
   return VT_OK;
 }
 

@@ -143,6 +143,13 @@ vt_status engine_upload_trace(vt_engine* e, const vt::DeviceLayout& layout, Scen
   return s;
 }
 
+uint32_t engine_trace_error(vt_engine* e, uint32_t word) {
+  if (e->fail_inject & kInjectTraceStack) word |= vtk::kErrorStack;
+  if (e->fail_inject & kInjectTraceGroup) word |= vtk::kErrorGroup;
+  e->fail_inject &= ~(kInjectTraceStack | kInjectTraceGroup);
+  return word;
+}
+
 vtk::DeviceScene engine_device_scene(const SceneBuffers& b, const vt::DeviceLayout& L, bool* wide) {
   vtk::DeviceScene d{};
   d.blas_nodes = (const float4*)b.blas.ptr;
@@ -557,9 +564,10 @@ static vt_status check_error_word(vt_engine* eng) {
   uint32_t err = 0;
   HIP_TRY(eng, hipMemcpyAsync(&err, eng->error_word.ptr, 4, hipMemcpyDeviceToHost, eng->stream));
   HIP_TRY(eng, hipStreamSynchronize(eng->stream));
+  err = engine_trace_error(eng, err);
   if (err) {
     (void)vtk::launch_zero((uint32_t*)eng->error_word.ptr, 1, eng->stream);
-    return set_err(eng, VT_ERR_HIP, "traversal stack capacity exceeded");
+    return set_err(eng, VT_ERR_HIP, vtk::trace_error_text(err));
   }
   return VT_OK;
 }

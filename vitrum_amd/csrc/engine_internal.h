@@ -64,8 +64,15 @@ struct RenderSceneData;  // one scene's shading data (render.cpp)
 
 // Test hooks (vt_debug_inject_failure): each bit makes the next matching step
 // fail once -- packing throws std::bad_alloc, the shading-data upload reports
-// an allocation failure, or its preparation throws std::runtime_error.
-enum : uint32_t { kInjectPackThrow = 1u, kInjectRenderAlloc = 2u, kInjectRenderThrow = 4u };
+// an allocation failure, or its preparation throws std::runtime_error; the
+// next check of the traversal's error word finds its stack or its group bit.
+enum : uint32_t {
+  kInjectPackThrow = 1u,
+  kInjectRenderAlloc = 2u,
+  kInjectRenderThrow = 4u,
+  kInjectTraceStack = 8u,
+  kInjectTraceGroup = 16u
+};
 struct CwbvhState;   // wide-BVH traversal buffers (cwbvh.cpp)
 struct RefitState;   // device refit buffers (refit.cpp)
 struct GpuBuildScratch;  // device BLAS builder buffers (gpubuild.cpp)
@@ -133,6 +140,8 @@ vt_status engine_upload_trace(vt_engine* e, const vt::DeviceLayout& layout, Scen
 // Device view of one scene's traversal buffers; `wide` reports whether its
 // Node128 trees can be walked (their worst-case stack fits the kernel's).
 vtk::DeviceScene engine_device_scene(const SceneBuffers& b, const vt::DeviceLayout& layout, bool* wide);
+// The traversal's error bits (traverse.h) with those a test hook adds.
+uint32_t engine_trace_error(vt_engine* e, uint32_t word);
 // Fills the scene and scheduling fields of a launch for the engine's scene.
 vtk::TraceParams engine_trace_params(vt_engine* e);
 // Packs, builds and uploads one scene's traversal buffers (engine.cpp).

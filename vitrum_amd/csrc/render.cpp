@@ -831,16 +831,17 @@ vt_status vt_capture(vt_engine* e, float* rgba, uint32_t width, uint32_t height)
     if (!rgba) return rerr(e, VT_ERR_INVALID_ARGUMENT, "rgba is NULL");
     if (!e->render || e->render->width != width || e->render->height != height)
       return rerr(e, VT_ERR_STATE, "no frame of this size has been rendered");
-    // The traversal's error word is read (and cleared) first: after a stack
-    // overflow the capture reports it once and leaves `rgba` untouched, and
-    // later captures succeed again.
+    // The traversal's error word is read (and cleared) first: after an error
+    // the capture reports it once and leaves `rgba` untouched, and later
+    // captures succeed again.
     uint32_t err = 0;
     HIP_CHECK(e, hipMemcpyAsync(&err, e->error_word.ptr, 4, hipMemcpyDeviceToHost, e->stream));
     HIP_CHECK(e, hipStreamSynchronize(e->stream));
+    err = engine_trace_error(e, err);
     if (err) {
       HIP_CHECK(e, vtk::launch_zero((uint32_t*)e->error_word.ptr, 1, e->stream));
       HIP_CHECK(e, hipStreamSynchronize(e->stream));
-      return rerr(e, VT_ERR_HIP, "traversal stack capacity exceeded during rendering");
+      return rerr(e, VT_ERR_HIP, std::string(vtk::trace_error_text(err)) + " during rendering");
     }
     HIP_CHECK(e, hipMemcpyAsync(rgba, e->render->accum.ptr, (size_t)width * height * 16,
                                 hipMemcpyDeviceToHost, e->stream));

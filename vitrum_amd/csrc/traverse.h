@@ -14,6 +14,12 @@ constexpr uint32_t kStackCapacity = 128;  // TLAS + BLAS entries per lane (>= 2 
 // their place), with the same spill area behind them.
 constexpr uint32_t kWideLdsDepth = kLdsDepth - 2;
 constexpr uint32_t kWideStackCapacity = kStackCapacity - 2;
+// Bits of a launch's error word: a lane's stack was full; the lanes of a wave
+// waited for helpers that were not there (wide_kernel).
+constexpr uint32_t kErrorStack = 1u, kErrorGroup = 2u;
+inline const char* trace_error_text(uint32_t bits) {
+  return bits & kErrorStack ? "traversal stack capacity exceeded" : "traversal waited for helpers that were not there";
+}
 // Wide nodes: children per node (a multiple of 4) and node size in float4s:
 // six coordinate rows and one child-ref row of kWideKids words, padded to
 // 8 rows (device_layout.h).
@@ -45,7 +51,7 @@ struct TraceParams {
   const uint32_t* n_ptr;  // when set, the ray count is read from device memory
   float* hit_pos;         // optional: world hit position, 3 floats per ray
   uint32_t* counter;   // work counter, zeroed by the launcher
-  uint32_t* error;     // set to non-zero on stack overflow
+  uint32_t* error;     // kError* bits, set by the kernel
   uint2* spill;        // (kStackCapacity - kLdsDepth) x grid threads
   uint32_t refill_min;    // refill a wave once this many lanes are idle
   uint32_t steps;         // traversal steps between refill checks

@@ -482,7 +482,7 @@ __global__ __launch_bounds__(BLOCK, 4) void trace_kernel(TraceParams p) {
 
   auto push = [&](uint32_t ref, float tn) {
     if (sp >= kStackCapacity) {
-      atomicOr(p.error, 1u);
+      atomicOr(p.error, kErrorStack);
       return false;
     }
     stk_store(sp++, make_uint2(ref, f2u(tn)));
@@ -1299,7 +1299,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         } else if (sp < kWideStackCapacity) {
           spill[(sp - D) * spill_stride + gtid] = (unsigned long long)ref | ((unsigned long long)f2u(tn) << 32);
         } else {
-          atomicOr(p.error, 1u);  // the host's bound rules this out
+          atomicOr(p.error, kErrorStack);  // the host's bound rules this out
           continue;
         }
         ++sp;
@@ -1376,7 +1376,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         if (HELP && all && (m_exit | m_enter | m_leaf) == 0ull) {
           // Only owners that wait, and no helper to wait for: cannot happen.
           // Report it and end the wave rather than wait for ever.
-          if (lane == 0) atomicOr(p.error, 2u);
+          if (lane == 0) atomicOr(p.error, kErrorGroup);
           mode = kIdle;
           break;
         }

@@ -369,7 +369,8 @@ class Engine:
     def inject_failure(self, flags):
         """Test hook: make the next vt_set_scene fail at the chosen step (bit
         1 packing throws std::bad_alloc, 2 the shading-data upload fails, 4
-        its preparation throws)."""
+        its preparation throws), or the next traversal check find an error (8 a
+        full stack, 16 a wave without its helpers)."""
         check(lib().vt_debug_inject_failure(self._h, C.c_uint32(flags)), self._h)
 
     def close(self):

@@ -371,7 +371,7 @@ vt_status vt_trace_any_device(vt_engine *eng, const vt_ray *d_rays, uint32_t n,
  * harnesses that forbid hipMalloc): it allocates nothing.  The launch's ray
  * counter, error word and stack-spill area live in a fixed 64 MiB device
  * array of the library (one copy per GPU, looked up at vt_create and held
- * until the process ends), which bounds the persistent grid at 606 blocks
+ * until the process ends), which bounds the persistent grid at 595 blocks
  * (512 on a 256-CU MI355X); rays and hits are the caller's.  Same hit
  * records as vt_trace_closest_device (binary / 4-wide walk; VT_ERR_STATE in
  * the cwbvh-closest mode); at most 2^31 - 1 rays per call (VT_ERR_RANGE).

@@ -2,7 +2,8 @@
 fill (one ray to more rays than lanes), so idle lanes walk subtrees of busy
 lanes' rays, against the oracle, bit for bit -- closest hit in each visiting
 order, any hit, and both with the path tracer's sided filter; and a scene of
-nearly coincident surfaces, whose near-ties a group has to walk again alone.
+nearly coincident surfaces, whose near-ties a group has to walk again alone;
+and stacks deeper than LDS holds.
 """
 import numpy as np
 import pytest
@@ -59,6 +60,51 @@ def test_every_fill_matches_oracle(engine, make):
                 assert np.array_equal(engine.trace_any(seg[:n]), want[sided][1][:n]), (n, sided)
     finally:
         engine.set_hit_filter(0)
+        engine.set_trace_tuning(8, 16, 2, 12)
+
+
+def _spine(near, far, ratio=1.5, seed=3):
+    """Clusters of three triangles at distances ratio^k along +x, `near` of
+    them in one mesh and each of the `far` others an instance: both trees are
+    spines, and a ray from the origin goes down all of them with a sibling
+    waiting at almost every level (86 entries at worst for 57 and 57)."""
+    rng = np.random.default_rng(seed)
+    n = near + far
+    tri = rng.normal(size=(n, 3, 3, 3)) * [0.02, 0.04, 0.04]
+    tri += rng.uniform(-0.25, 0.25, (n, 3, 1, 3)) * [0.2, 1.0, 1.0] + [1.0, 0.0, 0.0]
+    tri *= (ratio ** np.arange(n))[:, None, None, None]
+
+    def mesh(t):
+        v = t.reshape(-1, 3)
+        return W._mesh(v, np.tile([0, 1, 0], (len(v), 1)), np.arange(len(v), dtype=np.uint32).reshape(-1, 3), W.WHITE)
+
+    return {"primitives": [mesh(tri[:near])] + [mesh(t) for t in tri[near:]], "scene_radius": float(ratio ** n)}
+
+
+def test_deep_stacks_with_helpers(engine):
+    """Stacks well past the 18 entries in LDS, whose bottom entries are given
+    away and whose top is in the spill area."""
+    sc = _spine(57, 57)
+    engine.set_scene(sc)
+    ps = O.PackedScene(O.pack_scene([dict(p, material_id=i) for i, p in enumerate(sc["primitives"])]))
+    n, rng = 20000, np.random.default_rng(21)
+    rays = np.zeros(n, W.RAY_DTYPE)
+    d = np.concatenate([np.ones((n, 1)), rng.uniform(-0.22, 0.22, (n, 2))], 1)
+    rays["d"] = W._unit_f32(d.astype(np.float32))
+    rays["o"] = rng.uniform(-0.01, 0.01, (n, 3)).astype(np.float32)
+    rays["tmin"], rays["tmax"] = 1e-4, W.TMAX_INFINITY
+    ref, occ = O.trace_closest(ps, rays), O.trace_any(ps, rays)
+    assert np.unique(ref["inst"]).size > 20 and 0.5 < occ.mean() < 0.9
+    try:
+        for near in (0, 1, 2):
+            engine.set_trace_tuning(8, 16, near, 12)
+            for count in (1, 100, 4097, n):
+                got = engine.trace_closest(rays[:count])
+                for k in FIELDS:
+                    assert np.array_equal(got[k].view(np.uint32), ref[k][:count].view(np.uint32)), (near, count, k)
+        for count in (1, 100, 4097, n):
+            assert np.array_equal(engine.trace_any(rays[:count]), occ[:count]), count
+    finally:
         engine.set_trace_tuning(8, 16, 2, 12)
 
 

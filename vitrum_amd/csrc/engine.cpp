@@ -163,7 +163,7 @@ vtk::DeviceScene engine_device_scene(const SceneBuffers& b, const vt::DeviceLayo
   d.blas4_nodes = (const float4*)b.blas4.ptr;
   d.tlas4_nodes = (const float4*)b.tlas4.ptr;
   d.tlas4_root = L.tlas4_root;
-  if (wide) *wide = L.tlas_node_count != 0 && !L.blas4_nodes.empty() && L.stack4_need <= vtk::kWideStackCapacity;
+  if (wide) *wide = L.tlas_node_count != 0 && !L.blas4_nodes.empty() && L.stack4_need <= vtk::kStackCapacity;
   return d;
 }
 
@@ -277,8 +277,7 @@ vt_status vt_create(int32_t device_ordinal, const vt_options* opts, vt_engine** 
     e->trace_grid = e->cu_count * e->trace_blocks_per_cu;
     vt_status s = e->counter.ensure(e.get(), 64);
     if (!s) s = e->error_word.ensure(e.get(), 64);
-    const size_t spill = (size_t)(vtk::kStackCapacity - vtk::kLdsDepth) * e->trace_grid *
-                         vtk::kTraceBlock * sizeof(uint2);
+    const size_t spill = (size_t)vtk::kSpillDepth * e->trace_grid * vtk::kTraceBlock * sizeof(uint2);
     if (!s) s = e->spill.ensure(e.get(), spill);
     if (s) return set_err(nullptr, s, e->last_error);
     HIP_TRY(nullptr, vtk::launch_zero((uint32_t*)e->error_word.ptr, 16, e->stream));

@@ -17,9 +17,8 @@ namespace {
 // error word, then the stack-spill area from byte 256 on.
 constexpr size_t kScratchBytes = size_t(64) << 20;  // 64 MiB per device
 constexpr size_t kSpillOffset = 256;
-constexpr size_t kBlockSpillBytes =
-    (size_t)(vtk::kStackCapacity - vtk::kLdsDepth) * vtk::kTraceBlock * sizeof(uint2);  // 110,592
-constexpr uint32_t kMaxBlocks = (uint32_t)((kScratchBytes - kSpillOffset) / kBlockSpillBytes);  // 606
+constexpr size_t kBlockSpillBytes = (size_t)vtk::kSpillDepth * vtk::kTraceBlock * sizeof(uint2);  // 112,640
+constexpr uint32_t kMaxBlocks = (uint32_t)((kScratchBytes - kSpillOffset) / kBlockSpillBytes);  // 595
 constexpr int kMaxDevices = 64;
 
 std::mutex g_mutex;

@@ -764,7 +764,7 @@ vt_status vt_render_frame(vt_engine* e, const vt_frame* fr) {
     // previous bounce's shadow trace: each gets half of the persistent grid,
     // its own ray counter and its own half of the stack-spill area.
     const uint32_t half_grid = std::max(1u, e->trace_grid / 2u);
-    const size_t spill_half = (size_t)(vtk::kStackCapacity - vtk::kLdsDepth) * half_grid * vtk::kTraceBlock;
+    const size_t spill_half = (size_t)vtk::kSpillDepth * half_grid * vtk::kTraceBlock;
     for (uint32_t v = 0; v <= f.bounce_limit; ++v) {
       ps.queue = (uint32_t*)R.queue[cur].ptr;
       ps.rays = (float4*)R.rays[cur].ptr;

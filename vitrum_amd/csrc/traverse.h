@@ -11,9 +11,9 @@ constexpr uint32_t kTraceBlock = 128;     // threads per block (2 waves)
 constexpr uint32_t kLdsDepth = 20;        // stack entries per lane kept in LDS
 constexpr uint32_t kStackCapacity = 128;  // TLAS + BLAS entries per lane (>= 2 * 58 + 2)
 // The Node128 kernel keeps two entries fewer in LDS (its wave tables take
-// their place), with the same spill area behind them.
+// their place); the spill area holds what either keeps there.
 constexpr uint32_t kWideLdsDepth = kLdsDepth - 2;
-constexpr uint32_t kWideStackCapacity = kStackCapacity - 2;
+constexpr uint32_t kSpillDepth = kStackCapacity - kWideLdsDepth;  // entries per lane
 // Bits of a launch's error word: a lane's stack was full; the lanes of a wave
 // waited for helpers that were not there (wide_kernel).
 constexpr uint32_t kErrorStack = 1u, kErrorGroup = 2u;
@@ -52,7 +52,7 @@ struct TraceParams {
   float* hit_pos;         // optional: world hit position, 3 floats per ray
   uint32_t* counter;   // work counter, zeroed by the launcher
   uint32_t* error;     // kError* bits, set by the kernel
-  uint2* spill;        // (kStackCapacity - kLdsDepth) x grid threads
+  uint2* spill;        // kSpillDepth x grid threads
   uint32_t refill_min;    // refill a wave once this many lanes are idle
   uint32_t steps;         // traversal steps between refill checks
   uint32_t near_first;    // closest hit: visit the nearer child first (ties as the reference)

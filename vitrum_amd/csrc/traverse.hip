@@ -1296,7 +1296,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
         const float tn = c == 3 ? g3 : (c == 2 ? g2 : (c == 1 ? g1 : g0));
         if (sp < D) {
           stack[sp * B + tid] = make_uint2(ref, f2u(tn));
-        } else if (sp < kWideStackCapacity) {
+        } else if (sp < kStackCapacity) {
           spill[(sp - D) * spill_stride + gtid] = (unsigned long long)ref | ((unsigned long long)f2u(tn) << 32);
         } else {
           atomicOr(p.error, kErrorStack);  // the host's bound rules this out

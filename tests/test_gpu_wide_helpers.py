@@ -63,6 +63,74 @@ def test_every_fill_matches_oracle(engine, make):
         engine.set_trace_tuning(8, 16, 2, 12)
 
 
+FILL = 256 * 8 * 128  # rays of one static fill: 8 workgroups of 128 on every CU of an MI355X
+
+
+class _Device:
+    """Traces through device buffers that hold no answer beforehand."""
+
+    def __init__(self, engine, rays):
+        self.e, self.n = engine, rays.size
+        self.rays, self.out = engine.alloc(rays.nbytes), engine.alloc(rays.size * W.HIT_DTYPE.itemsize)
+        engine.h2d(self.rays, rays)
+
+    def close(self):
+        self.e.free(self.rays)
+        self.e.free(self.out)
+
+    def _run(self, call, n, dtype):
+        got = np.frombuffer(b"\x5a" * (n * np.dtype(dtype).itemsize), dtype).copy()
+        self.e.h2d(self.out, got)
+        call(self.rays, n, self.out)
+        self.e.synchronize()
+        self.e.d2h(got, self.out)
+        return got
+
+    def closest(self, n):
+        return self._run(self.e.trace_closest_device, n, W.HIT_DTYPE)
+
+    def any(self, n):
+        return self._run(self.e.trace_any_device, n, np.uint32)
+
+
+# Few triangles an instance and many: any-hit launches end in another order.
+@pytest.mark.parametrize("make", [lambda: W.cornell_scene(2048), _box], ids=["small_meshes", "large_meshes"])
+def test_past_the_static_fill_matches_oracle(engine, make):
+    """More rays than the grid's lanes: waves fetch from the counter, without
+    helpers until the supply ends, with a transposed end that is a part of the
+    queue (first size) or its largest (second)."""
+    sc = make()
+    engine.set_scene(sc)
+    pack = O.pack_scene([dict(p, material_id=i) for i, p in enumerate(sc["primitives"])])
+    ps = O.PackedScene(pack)
+    rays, st = W.primary_rays(sc["camera"], 128, 128, scene_radius=sc["scene_radius"])
+    rays = np.concatenate([rays, W.bounce_rays(pack, rays, O.trace_closest(ps, rays), st, sc["scene_radius"])])
+    rays = rays[np.random.default_rng(19).permutation(rays.size)]
+    seg = rays.copy()
+    seg["tmax"] = np.random.default_rng(20).uniform(0.05, 3.0, rays.size).astype(np.float32)
+    flags = O.single_sided_flags(ps, [p["material"] for p in sc["primitives"]])
+    sizes = (FILL + 4097, 3 * FILL + 777)
+    want = {0: (O.trace_closest(ps, rays), O.trace_any(ps, seg)),
+            1: (O.trace_closest_sided(ps, flags, rays), O.trace_occluded_sided(ps, flags, seg))}
+    dev, dseg = _Device(engine, np.resize(rays, sizes[-1])), _Device(engine, np.resize(seg, sizes[-1]))
+    try:
+        for n in sizes:
+            for sided in (0, 1):
+                engine.set_hit_filter(sided)
+                hits = np.resize(want[sided][0], n)
+                for near in (0, 1, 2):
+                    engine.set_trace_tuning(8, 16, near, 12)
+                    got = dev.closest(n)
+                    for k in FIELDS:
+                        assert np.array_equal(got[k].view(np.uint32), hits[k].view(np.uint32)), (n, sided, near, k)
+                assert np.array_equal(dseg.any(n), np.resize(want[sided][1], n)), (n, sided)
+    finally:
+        engine.set_hit_filter(0)
+        engine.set_trace_tuning(8, 16, 2, 12)
+        dev.close()
+        dseg.close()
+
+
 def _spine(near, far, ratio=1.5, seed=3):
     """Clusters of three triangles at distances ratio^k along +x, `near` of
     them in one mesh and each of the `far` others an instance: both trees are

@@ -1039,6 +1039,13 @@ __device__ __forceinline__ float4 load4(const float4* p) {
 // 35.8, 34.7, 33.6 and 33.8 ms, shadow rays in the box 1.08 (0) and 0.59 ms
 // (128); the 1M-triangle scene, whose nodes fit no cache, 0.950, 0.956, 0.967
 // and 1.095 ms.  The 256 x 256 frame below: 2.73 -> 2.13 ms.
+// Any hits among small meshes have no long rays, and lose the coherence for
+// nothing: below 1,024 triangles an instance their queues end in order.  Any
+// hits of 1024 x 1024 primary rays and of shadow rays, transposed and in
+// order: 8,192 boxes of 12 triangles 558 -> 483 and 584 -> 511 us, the box at
+// 256 triangles an instance 244 -> 227 and 248 -> 232, at 512 251 -> 234 and
+// 292 -> 304, at 1,024 272 -> 257 and 385 -> 439, at 4,096 311 -> 291 and
+// 875 -> 1,060 us.
 //
 // Measured against the same walk without these three (trace_kernel over
 // Node128): 1,677,721 rays of the 1M-triangle scene 1.27 -> 0.97 ms;
@@ -1065,6 +1072,7 @@ constexpr uint32_t kfAlone = 8192u;    // no helpers in this instance (walked ag
 constexpr uint32_t kfLocal = kfLevel | kfMirror | kfLHit | kfLFront | kfLSingle | kfSplit | kfTie;
 constexpr uint32_t kHelpSteps = 4;     // steps between two rounds of taking work
 constexpr uint32_t kTailRays = 128;    // per wave, of a queue's end
+constexpr uint32_t kTailMesh = 1024;   // triangles an instance, for any hits
 
 // Orders a wave's LDS accesses of different lanes (they execute in program
 // order; this keeps the compiler from moving them).
@@ -1099,7 +1107,8 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wide_kernel(TraceParams p) {
   // fill covers them all, and the last `tail` of a longer queue transposed.
   const bool one_fill = static_end >= n_rays;
   const uint32_t far = take_cap < 64u ? n_waves : 1u;
-  const uint32_t tail = one_fill ? 0u : min(n_waves * kTailRays, n_rays - static_end) & ~63u;
+  const bool in_order = ANY && !MULTI && p.scene.tri_count / kTailMesh < p.scene.inst_count;
+  const uint32_t tail = one_fill || in_order ? 0u : min(n_waves * kTailRays, n_rays - static_end) & ~63u;
   const uint32_t tail_begin = n_rays - tail;
 
   uint32_t mode = kIdle, fl = 0, ray_idx = 0, sid = 0;

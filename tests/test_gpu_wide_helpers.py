@@ -1,9 +1,9 @@
 """The Node128 traversal kernel where its waves share work: launches of every
-fill (one ray to more rays than lanes), so idle lanes walk subtrees of busy
-lanes' rays, against the oracle, bit for bit -- closest hit in each visiting
-order, any hit, and both with the path tracer's sided filter; and a scene of
-nearly coincident surfaces, whose near-ties a group has to walk again alone;
-and stacks deeper than LDS holds.
+fill (one ray to several rays for each lane of the grid), so idle lanes walk
+subtrees of busy lanes' rays, against the oracle, bit for bit -- closest hit
+in each visiting order, any hit, and both with the path tracer's sided filter;
+a scene of nearly coincident surfaces, whose near-ties a group has to walk
+again alone; stacks deeper than LDS holds; and rays that are not finite.
 """
 import numpy as np
 import pytest
@@ -48,7 +48,8 @@ def test_every_fill_matches_oracle(engine, make):
             1: (O.trace_closest_sided(ps, flags, rays), O.trace_occluded_sided(ps, flags, seg))}
     try:
         # one ray; a wave less and more than full; every wave one ray; a few
-        # rays each; about a full static fill; refills from the counter
+        # rays each; half of a full static fill (every wave helps from its
+        # first step)
         for n in (1, 63, 64, 65, 4095, 16411, 70001, rays.size):
             for sided in (0, 1):
                 engine.set_hit_filter(sided)
@@ -176,6 +177,53 @@ def test_deep_stacks_with_helpers(engine):
         engine.set_trace_tuning(8, 16, 2, 12)
 
 
+def test_rays_that_are_not_finite(engine):
+    """NaN, infinite, zero, denormal and huge components among usual rays:
+    the records of the binary walk and of the oracle."""
+    sc = W.cornell_scene(2048)
+    engine.set_scene(sc)
+    ps = O.PackedScene(O.pack_scene([dict(p, material_id=i) for i, p in enumerate(sc["primitives"])]))
+    n, rng = 24000, np.random.default_rng(22)
+    rays = np.zeros(n, W.RAY_DTYPE)
+    rays["o"] = (np.array([0, 1, 0]) + rng.uniform(-0.9, 0.9, (n, 3))).astype(np.float32)
+    rays["d"] = W._unit_f32(rng.normal(size=(n, 3)).astype(np.float32))
+    rays["tmin"], rays["tmax"] = 1e-4, W.TMAX_INFINITY
+    kind, axis = np.arange(n) % 24, np.arange(n) // 24 % 3
+    odd = [("o", np.nan), ("o", np.inf), ("o", 3e38), ("d", np.nan), ("d", np.inf), ("d", -np.inf), ("d", 0.0), ("d", -0.0),
+           ("d", 1e-45), ("d", 3e38), ("tmin", np.nan), ("tmin", np.inf), ("tmin", -1.0), ("tmax", np.nan),
+           ("tmax", np.inf), ("tmax", 0.0)]
+    for j, (field, value) in enumerate(odd):
+        m = kind == j
+        if rays[field].ndim == 2:
+            rays[field][m, axis[m]] = value
+        else:
+            rays[field][m] = value
+    m = (kind >= 6) & (kind <= 8)  # unit directions again, along an axis plane
+    rays["d"][m] = np.where(np.abs(rays["d"][m]) <= 1e-45, rays["d"][m], W._unit_f32(rays["d"][m]))
+    rays["d"][kind == 16] = 0.0
+    rays["d"][kind == 17] *= np.float32(1e-30)
+    rays["d"][kind == 18] *= np.float32(1e20)
+    ref = O.trace_closest(ps, rays)
+    try:
+        for sided in (0, 1):
+            engine.set_hit_filter(sided)
+            for near in (0, 1, 2):
+                engine.set_trace_tuning(8, 16, near, 12)
+                got = {}
+                for width in (2, 4):
+                    engine.set_node_width(width)
+                    got[width] = engine.trace_closest(rays), engine.trace_any(rays)
+                for k in FIELDS:
+                    assert np.array_equal(got[4][0][k].view(np.uint32), got[2][0][k].view(np.uint32)), (sided, near, k)
+                    if not sided:
+                        assert np.array_equal(got[4][0][k].view(np.uint32), ref[k].view(np.uint32)), (near, k)
+                assert np.array_equal(got[4][1], got[2][1]), (sided, near)
+    finally:
+        engine.set_hit_filter(0)
+        engine.set_node_width(4)
+        engine.set_trace_tuning(8, 16, 2, 12)
+
+
 def _grazing(n, seed):
     """A yawed box and rays that meet its faces at 1e-7 to 1e-2 rad, most near
     the edges and vertices of the grid: hits shared by two triangles and
@@ -207,6 +255,11 @@ def test_grazing_hits_do_not_depend_on_the_group(engine):
         for near in (0, 1, 2):
             engine.set_trace_tuning(8, 16, near, 12)
             first = engine.trace_closest(rays)
+            # 64 copies of a ray fill a wave and end together: no lane helps
+            waves = FILL // 64
+            for lo in range(0, 2 * waves, waves):
+                alone = engine.trace_closest(np.repeat(rays[lo:lo + waves], 64))
+                assert np.array_equal(np.repeat(first[lo:lo + waves], 64).view(np.uint8), alone.view(np.uint8)), near
             if near == 0:  # the reference's order is exact, ties included
                 ref = O.trace_closest(ps, rays)
                 for k in FIELDS:
@@ -226,10 +279,12 @@ def test_every_ray_is_handed_out_once(engine, extra):
     sc = W.cornell_scene(2048)
     engine.set_scene(sc)
     one = W.primary_rays(sc["camera"], 64, 64)[0]
-    for base in (8192, 262144):
+    hits, occ = engine.trace_closest(one), engine.trace_any(one)
+    for base in (FILL // 32, FILL):
         n = base + extra
-        rays = np.resize(one, n)
-        want = np.resize(engine.trace_closest(one), n)
-        assert np.array_equal(engine.trace_closest(rays).view(np.uint8), want.view(np.uint8)), n
-        occ = engine.trace_any(rays)
-        assert np.array_equal(occ, np.resize(engine.trace_any(one), n)), n
+        dev = _Device(engine, np.resize(one, n))
+        try:
+            assert np.array_equal(dev.closest(n).view(np.uint8), np.resize(hits, n).view(np.uint8)), n
+            assert np.array_equal(dev.any(n), np.resize(occ, n)), n
+        finally:
+            dev.close()

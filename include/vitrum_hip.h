@@ -447,6 +447,10 @@ vt_status vt_set_bvh_traversal(vt_engine *eng, uint32_t mode);
  * square root round exactly like the host's. Host buffers. */
 vt_status vt_selftest_fp32(vt_engine *eng, const float *a, const float *b, float *q, float *r,
                            uint32_t n);
+/* Test hook: q = a / b as the traversal and the light tree divide several
+ * numerators by one denominator, l = log2(b) as the light tree takes it. */
+vt_status vt_selftest_math(vt_engine *eng, const float *a, const float *b, float *q, float *l,
+                           uint32_t n);
 
 /* ---- device memory and stream plumbing ----------------------------------- */
 

@@ -17,6 +17,7 @@
 #include "device_layout.h"
 #include "engine_internal.h"
 #include "gpubuild.h"
+#include "render.h"
 #include "traverse.h"
 
 namespace {
@@ -659,25 +660,34 @@ vt_status vt_set_trace_tuning(vt_engine* eng, uint32_t refill_min, uint32_t step
   });
 }
 
+// Two arrays through a selftest kernel and its two results back.
+static vt_status selftest(vt_engine* eng, const float* a, const float* b, float* q, float* r, uint32_t n,
+                          hipError_t (*launch)(const float*, const float*, float*, float*, uint32_t, hipStream_t)) {
+  if (!eng || (n && (!a || !b || !q || !r)))
+    return set_err(eng, VT_ERR_INVALID_ARGUMENT, "NULL argument");
+  if (n == 0) return VT_OK;
+  HIP_TRY(eng, hipSetDevice(eng->device));
+  DeviceBuffer buf;
+  if (vt_status s = buf.ensure(eng, (size_t)n * 16)) return s;
+  float* d = (float*)buf.ptr;
+  HIP_TRY(eng, hipMemcpyAsync(d, a, (size_t)n * 4, hipMemcpyHostToDevice, eng->stream));
+  HIP_TRY(eng, hipMemcpyAsync(d + n, b, (size_t)n * 4, hipMemcpyHostToDevice, eng->stream));
+  HIP_TRY(eng, launch(d, d + n, d + 2 * (size_t)n, d + 3 * (size_t)n, n, eng->stream));
+  HIP_TRY(eng, hipMemcpyAsync(q, d + 2 * (size_t)n, (size_t)n * 4, hipMemcpyDeviceToHost, eng->stream));
+  HIP_TRY(eng, hipMemcpyAsync(r, d + 3 * (size_t)n, (size_t)n * 4, hipMemcpyDeviceToHost, eng->stream));
+  HIP_TRY(eng, hipStreamSynchronize(eng->stream));
+  buf.release();
+  return VT_OK;
+}
+
 vt_status vt_selftest_fp32(vt_engine* eng, const float* a, const float* b, float* q, float* r,
                            uint32_t n) {
-  return vt_guarded(eng, [&]() -> vt_status {
-    if (!eng || (n && (!a || !b || !q || !r)))
-      return set_err(eng, VT_ERR_INVALID_ARGUMENT, "NULL argument");
-    if (n == 0) return VT_OK;
-    HIP_TRY(eng, hipSetDevice(eng->device));
-    DeviceBuffer buf;
-    if (vt_status s = buf.ensure(eng, (size_t)n * 16)) return s;
-    float* d = (float*)buf.ptr;
-    HIP_TRY(eng, hipMemcpyAsync(d, a, (size_t)n * 4, hipMemcpyHostToDevice, eng->stream));
-    HIP_TRY(eng, hipMemcpyAsync(d + n, b, (size_t)n * 4, hipMemcpyHostToDevice, eng->stream));
-    HIP_TRY(eng, vtk::launch_fp32_selftest(d, d + n, d + 2 * (size_t)n, d + 3 * (size_t)n, n, eng->stream));
-    HIP_TRY(eng, hipMemcpyAsync(q, d + 2 * (size_t)n, (size_t)n * 4, hipMemcpyDeviceToHost, eng->stream));
-    HIP_TRY(eng, hipMemcpyAsync(r, d + 3 * (size_t)n, (size_t)n * 4, hipMemcpyDeviceToHost, eng->stream));
-    HIP_TRY(eng, hipStreamSynchronize(eng->stream));
-    buf.release();
-    return VT_OK;
-  });
+  return vt_guarded(eng, [&] { return selftest(eng, a, b, q, r, n, vtk::launch_fp32_selftest); });
+}
+
+vt_status vt_selftest_math(vt_engine* eng, const float* a, const float* b, float* q, float* l,
+                           uint32_t n) {
+  return vt_guarded(eng, [&] { return selftest(eng, a, b, q, l, n, vtr::launch_math_selftest); });
 }
 
 // ---------------------------------------------------------------------------

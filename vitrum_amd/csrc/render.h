@@ -132,6 +132,9 @@ struct PathState {
 hipError_t launch_light_prepare(const float* tree, uint32_t nodes, float4* out, hipStream_t st);
 // cos(theta) at the h + 1 row edges of an environment map; once per scene.
 hipError_t launch_env_rows(uint32_t h, double* out, hipStream_t st);
+// q = a / b by the division of fast_div.h where its conditions hold, and
+// l = the light tree's log2 of b (test hook).
+hipError_t launch_math_selftest(const float* a, const float* b, float* q, float* l, uint32_t n, hipStream_t st);
 hipError_t launch_camera(const FrameParams& f, const PathState& s, hipStream_t st);
 hipError_t launch_shade(const FrameParams& f, const ShadeScene& sc, const PathState& s,
                         uint32_t vertex, uint32_t capacity, hipStream_t st);

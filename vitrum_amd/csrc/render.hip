@@ -1907,6 +1907,20 @@ hipError_t launch_env_rows(uint32_t h, double* out, hipStream_t st) {
   return hipGetLastError();
 }
 
+__global__ void math_selftest_kernel(const float* a, const float* b, float* q, float* l, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float x = a[i], y = b[i];
+  const bool fast = vtd::div_den(y) && vtd::div_key(x) >= vtd::kDivNum && fabsf(x) < 0x1p80f;
+  q[i] = fast ? vtd::div_by(x, y, vtd::recip_of(y)) : x / y;
+  l[i] = lt_log2(y);
+}
+
+hipError_t launch_math_selftest(const float* a, const float* b, float* q, float* l, uint32_t n, hipStream_t st) {
+  hipLaunchKernelGGL(math_selftest_kernel, dim3((n + 255) / 256), dim3(256), 0, st, a, b, q, l, n);
+  return hipGetLastError();
+}
+
 hipError_t launch_camera(const FrameParams& f, const PathState& s, hipStream_t st) {
   const uint32_t n = f.pixels + (f.nrc ? f.train_paths : 0u);
   if (f.sobol)

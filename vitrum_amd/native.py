@@ -26,7 +26,7 @@ STATUS = {0: "VT_OK", -1: "VT_ERR_INVALID_ARGUMENT", -2: "VT_ERR_RANGE", -3: "VT
 EXPORTED = [
     "vt_create", "vt_destroy", "vt_last_error", "vt_set_scene", "vt_trace_closest", "vt_trace_any",
     "vt_trace_closest_device", "vt_trace_any_device", "vt_set_counting", "vt_trace_closest_counts",
-    "vt_set_trace_tuning", "vt_selftest_fp32", "vt_device_alloc", "vt_device_free",
+    "vt_set_trace_tuning", "vt_selftest_fp32", "vt_selftest_math", "vt_device_alloc", "vt_device_free",
     "vt_memcpy_h2d", "vt_memcpy_d2h", "vt_memcpy_d2d", "vt_synchronize", "vt_get_stream", "vt_stats",
     "vt_build_blas", "vt_build_tlas", "vt_pack_scene", "vt_pack_field_words",
     "vt_pack_copy_field", "vt_pack_free", "vt_version", "vt_render_frame", "vt_capture",
@@ -464,6 +464,17 @@ class Engine:
     def set_trace_tuning(self, refill_min, steps, near_first=2, defer_min=12):
         check(lib().vt_set_trace_tuning(self._h, C.c_uint32(refill_min), C.c_uint32(steps),
                                         C.c_uint32(near_first), C.c_uint32(defer_min)), self._h)
+
+    def selftest_math(self, a, b):
+        """(a / b as the traversal and the light tree divide by a shared
+        denominator, log2 b as the light tree takes it)."""
+        a = np.ascontiguousarray(a, np.float32)
+        b = np.ascontiguousarray(b, np.float32)
+        q = np.zeros_like(a)
+        r = np.zeros_like(a)
+        check(lib().vt_selftest_math(self._h, _p(a, F32P), _p(b, F32P), _p(q, F32P), _p(r, F32P),
+                                     C.c_uint32(a.size)), self._h)
+        return q, r
 
     def selftest_fp32(self, a, b):
         a = np.ascontiguousarray(a, np.float32)

@@ -592,7 +592,6 @@ __global__ __launch_bounds__(256, 2) void train_kernel(const float* __restrict__
     store_block(HT, at, B);
 #pragma unroll
     for (uint32_t l = 0; l < kHidden; ++l) {
-      // one layer's fragments at a time: loads are not hoisted across layers
       mask[l] = hidden_block(fw + l * kFragsHidden, lane, B);
       store_block(HT + (l + 1u) * kTile, at, B);
     }

@@ -1217,12 +1217,16 @@ __global__ void camera_kernel(FrameParams f0, PathState s) {
 // looked up at one place; rarely reached functions (pow, cos and sin in
 // binary64) are calls.  The kernel is built per sampler and with or without
 // the extension lobes (clearcoat, sheen, anisotropy), so that the usual scene
-// carries neither.  That took it from 276 registers (one wave per SIMD) to
-// 128.  One workgroup shades 256 entries and takes its places in the next
-// queues with one addition each.
-// Measured, with the same images (start, three and four waves per SIMD): a
+// carries neither.  It had 276 registers (one wave per SIMD); held to 128 the
+// four builds spill 44 to 67 of them (176 to 224 bytes of scratch a lane).
+// Held to 168, three waves per SIMD, they spill at most 12 and are as fast.
+// One workgroup shades 256 entries and takes its places in the next queues
+// with one addition each.
+// Measured, with the same images (before, three and four waves per SIMD): a
 // 1080p frame of the box 48.5, 38.5 and 37.6 ms; the 1M-triangle scene, Sobol
-// sampler and sky 9.5, 7.75 and 7.7 ms.
+// sampler and sky 9.5, 7.75 and 7.7 ms; a 1280 x 720 frame of the box with all
+// extension lobes 12.7, 4.65 and 4.61 ms (PCG) and 13.2, 4.71 and 4.77 ms
+// (Sobol), before including the traversal without helpers.
 constexpr int kShadeWaves = 4;
 
 // Material sort (f.shade_sort).  Each workgroup shades its 256 queue entries

@@ -13,8 +13,8 @@
 //
 // Design (MI355X):
 //  * wide_kernel walks Node128 trees (four child boxes per node); scenes
-//    whose Node128 stack bound is too deep, and the work counters, take
-//    trace_kernel.
+//    whose Node128 stack bound is too deep or that hold no instance, and the
+//    work counters, take trace_kernel.
 //  * Node64 BVH2 nodes: the two child boxes sit in the parent, so a node
 //    expansion is one 64-byte load and two slab tests.  The traversal order
 //    is the reference's left-first depth-first order; a child's entry

@@ -337,11 +337,11 @@ __device__ __forceinline__ void output_layer(const uint4* __restrict__ frags, ui
 //
 // Bound by VALU issue, with the LDS gathers and MFMAs behind it: a tile takes
 // 2,370 vector instructions beside 136 MFMAs (4,550 with the bf16 rounding
-// written out, eight exponentials a lane and flat gathers; 2,080 and 3% less
-// time with fused grid sums, a quotient corrected once and a shorter
+// written out, eight exponentials a lane and flat gathers; 2,080 and 3 to 5%
+// less time with fused grid sums, a quotient corrected once and a shorter
 // exponential, which changed the last bits of what the cache answers).
-// 2,073,600 samples: 286 -> 185 us.  Blocks of 512 threads (twice the registers, two
-// waves per SIMD) take 217 us.
+// 2,073,600 samples: 286 -> 185 us.  Blocks of 512 threads (twice the
+// registers, two waves per SIMD) took 217 us where these took 180.
 
 __global__ __launch_bounds__(kInferBlock) void infer_kernel(const float* __restrict__ feats, uint32_t cap,
                                                      const uint32_t* __restrict__ n_ptr,
